@@ -59,7 +59,7 @@ template <typename T> struct BatchImpl {
         size_t map_off = 0;            // into maps
         size_t pass_off = 0;           // into passes (FFT stages)
         size_t lds = 0;
-        int max_elems = 0;             // largest C * L of an FFT stage
+        bool fft_line = false;         // register-resident passes (FFT stages)
     };
 
     int d = 0, m = 0, W = 0, R = 0;
@@ -307,27 +307,32 @@ template <typename T> struct BatchImpl {
             }
             L.nblk = (uint32_t)(mh.size() - L.map_off);
         };
+        // one launch for the register-resident passes and, where a job's line length
+        // has none, one for the generic passes
         auto add_fft = [&](int dir, int t) {
-            Launch L;
-            L.fft_t = t;
-            L.pass_off = ph.size();
-            L.map_off = mh.size();
-            for (int i = 0; i < P; ++i) {
-                const Prob &p = probs[i];
-                for (int r = 0; r < R; ++r) {
-                    const FftLaunch<T> f = fft_pass_setup<T>(
-                        p.ge, static_cast<const C *>(p.ft->tw[t]), p.roc, p.rocoff, t, dir == 0,
-                        p.fhat_in + (size_t)r * p.N_total, p.fhat_out + (size_t)r * p.N_total,
-                        p.g + (size_t)r * p.n_total);
-                    const uint32_t job = (uint32_t)(ph.size() - L.pass_off);
-                    ph.push_back(f.P);
-                    for (int64_t k = 0; k < f.blocks; ++k) mh.push_back(BlockMap{job, (uint32_t)k});
-                    L.lds = std::max(L.lds, f.lds);
-                    L.max_elems = std::max(L.max_elems, f.P.C * f.P.L);
+            for (const bool line : {true, false}) {
+                Launch L;
+                L.fft_t = t;
+                L.fft_line = line;
+                L.pass_off = ph.size();
+                L.map_off = mh.size();
+                for (int i = 0; i < P; ++i) {
+                    const Prob &p = probs[i];
+                    for (int r = 0; r < R; ++r) {
+                        const FftLaunch<T> f = fft_pass_setup<T>(
+                            p.ge, static_cast<const C *>(p.ft->tw[t]), p.roc, p.rocoff, t, dir == 0,
+                            p.fhat_in + (size_t)r * p.N_total, p.fhat_out + (size_t)r * p.N_total,
+                            p.g + (size_t)r * p.n_total, FFT_BATCH);
+                        if ((f.P.tpl > 0) != line) break;   // the problem's other launch
+                        const uint32_t job = (uint32_t)(ph.size() - L.pass_off);
+                        ph.push_back(f.P);
+                        for (int64_t k = 0; k < f.blocks; ++k) mh.push_back(BlockMap{job, (uint32_t)k});
+                        L.lds = std::max(L.lds, f.lds);
+                    }
                 }
+                L.nblk = (uint32_t)(mh.size() - L.map_off);
+                if (L.nblk > 0) stages[dir].push_back(L);
             }
-            L.nblk = (uint32_t)(mh.size() - L.map_off);
-            stages[dir].push_back(L);
         };
         auto add_grid = [&](int dir, BatchStage st, auto blocks) {
             Launch L;
@@ -377,9 +382,11 @@ template <typename T> struct BatchImpl {
     void launch_stages(int dir, hipStream_t s)
     {
         for (const Launch &L : stages[dir]) {
-            if (L.fft_t >= 0)
-                launch_fft_batch<T>(passes + L.pass_off, maps + L.map_off, L.nblk, L.lds,
-                                    L.max_elems, s);
+            if (L.fft_t >= 0 && L.fft_line)
+                launch_fft_line_batch<T>(passes + L.pass_off, maps + L.map_off, L.nblk, L.fft_t == d - 1,
+                                         L.lds, s);
+            else if (L.fft_t >= 0)
+                launch_fft_batch<T>(passes + L.pass_off, maps + L.map_off, L.nblk, L.lds, s);
             else
                 launch_batch_stage<T>(L.st, jobs[L.dir], maps + L.map_off, L.nblk, d, W,
                                       config[dir], s);

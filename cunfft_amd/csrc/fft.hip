@@ -5,34 +5,39 @@
 //            src/cunfft_wrapper.cu:32-75)  then cufftExec(.., CUFFT_FORWARD)
 //   adjoint  cufftExec(.., CUFFT_INVERSE) then kernelRollOf_adjoint_{1,2,3}d
 //            (src/cunfft_kernel.cu:264-467, src/cunfft_wrapper.cu:77-121)
-// A d-dimensional transform is d passes, one per axis.  Each workgroup loads
-// C whole lines of the axis into LDS, runs radix-4 (and one radix-2) Stockham
-// stages there -- then radix-3 stages when L = 2^a 3^b is not a power of two
-// -- and writes the lines back: one HBM read and one write per pass.  The forward passes skip lines that are still all zero and read only
-// the N_t nonzero entries of each line; the first forward pass reads fhat and
-// applies exp(fac k^2) on the way in.  The adjoint passes write only the N_t
-// entries that survive the crop; the last one writes fhat with exp(fac k^2).
-// Twiddles come from a per-length table computed in extended precision on
-// the host.
+// A d-dimensional transform is d passes, one per axis, each one HBM read and
+// one write.  The forward passes skip lines that are still all zero and read
+// only the N_t nonzero entries of each line; the first forward pass reads fhat
+// and applies exp(fac k^2) on the way in.  The adjoint passes write only the
+// N_t entries that survive the crop; the last one writes fhat with exp(fac k^2).
+// Twiddles come from a per-length table computed in extended precision on the
+// host.
+//
+// The usual line lengths (8 .. 4096 powers of two, 3 2^k and 9 2^k up to 1536)
+// run the register-resident pass of fft_line.hpp.  This file holds the set-up
+// of the passes and the generic pass for the other lengths 2^a 3^b: each
+// workgroup loads C whole lines into LDS, runs Stockham stages there and writes
+// the lines back.
 #include <algorithm>
 #include <type_traits>
 
-#include "internal.hpp"
+#include "fft_line.hpp"
 
 namespace cunfft {
 
+// (instantiated in fft_line_f32.hip and fft_line_f64.hip)
+extern template void launch_fft_line<float>(const FftPass<float> &, int64_t, size_t, hipStream_t);
+extern template void launch_fft_line<double>(const FftPass<double> &, int64_t, size_t, hipStream_t);
+
 constexpr int kFftThreads = 256;
-// Elements C * L per workgroup: up to 4096 (an 8192-element FP32 variant,
-// for 16 columns of a 512-point column pass, measured slower and was
-// dropped).  The kernels hold E / 1024 radix-4 butterflies per thread in
-// registers.
-template <typename T> constexpr int fft_max_elems() { return 4096; }
-constexpr int kFftSmallElems = 4096;
+// Elements C * L per workgroup of the generic pass: up to kFftElems.
+constexpr int kFftElems = 4096;
 // global loads in flight per thread from fhat (FP64: fewer, the registers run
 // short); loads from the grid, with no FP64 roll-off factor to hold, take twice
 // as many (FP64 3D 256^3 passes 3% faster, FP32 unchanged)
 template <typename T> constexpr int fft_load_batch() { return sizeof(T) == 4 ? 8 : 4; }
 constexpr int kMaxRowsPerGroup = 64;
+constexpr int kFftLineLds = 144 * 1024;   // LDS of a register-resident pass's lines, at most
 
 template <typename T>
 __device__ __forceinline__ cplx_t<T> cmul(const cplx_t<T> a, const cplx_t<T> b)
@@ -100,178 +105,6 @@ __device__ LineInfo line_info(const FftPass<T> &P, int64_t pa)
     li.fbase = fq * (P.t == 0 ? P.N[0] : (P.t == 1 ? P.N[1] : P.N[2]));
     li.fac = fac;
     return li;
-}
-
-template <typename T, int E>
-__device__ __forceinline__ void stage4(cplx_t<T> *buf, const cplx_t<T> *__restrict__ tw, int logL,
-                                       int C, int ldsL, int logNs, int sign, int tid)
-{
-    const int logQ = logL - 2;
-    const int Q = 1 << logQ;
-    const int Ns = 1 << logNs;
-    const int nb = C << logQ;
-    constexpr int kMaxB4 = E / 4 / kFftThreads;
-    cplx_t<T> v[kMaxB4][4];
-#pragma unroll
-    for (int k = 0; k < kMaxB4; ++k) {
-        const int b = tid + k * kFftThreads;
-        if (b < nb) {
-            const int c = b >> logQ, j = b & (Q - 1);
-            const cplx_t<T> *base = buf + c * ldsL + j;
-            v[k][0] = base[0];
-            v[k][1] = base[Q];
-            v[k][2] = base[2 * Q];
-            v[k][3] = base[3 * Q];
-            if (Ns > 1) {
-                const int step = (j & (Ns - 1)) << (logL - 2 - logNs);
-                v[k][1] = cmul<T>(v[k][1], twiddle<T>(tw, step, sign));
-                v[k][2] = cmul<T>(v[k][2], twiddle<T>(tw, 2 * step, sign));
-                v[k][3] = cmul<T>(v[k][3], twiddle<T>(tw, 3 * step, sign));
-            }
-            dft4<T>(v[k], sign);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kMaxB4; ++k) {
-        const int b = tid + k * kFftThreads;
-        if (b < nb) {
-            const int c = b >> logQ, j = b & (Q - 1);
-            const int out = ((j >> logNs) << (logNs + 2)) + (j & (Ns - 1));
-            cplx_t<T> *ob = buf + c * ldsL + out;
-            ob[0] = v[k][0];
-            ob[Ns] = v[k][1];
-            ob[2 * Ns] = v[k][2];
-            ob[3 * Ns] = v[k][3];
-        }
-    }
-    __syncthreads();
-}
-
-// Final radix-2 stage (Ns = L/2): butterfly j combines j and j + L/2 in place.
-template <typename T, int E>
-__device__ __forceinline__ void stage2_last(cplx_t<T> *buf, const cplx_t<T> *__restrict__ tw,
-                                            int logL, int C, int ldsL, int sign, int tid)
-{
-    const int logH = logL - 1;
-    const int H = 1 << logH;
-    const int nb = C << logH;
-    constexpr int kMaxB2 = E / 2 / kFftThreads;
-#pragma unroll
-    for (int k = 0; k < kMaxB2; ++k) {
-        const int b = tid + k * kFftThreads;
-        if (b < nb) {
-            const int c = b >> logH, j = b & (H - 1);
-            cplx_t<T> *base = buf + c * ldsL + j;
-            const cplx_t<T> v0 = base[0];
-            const cplx_t<T> v1 = cmul<T>(base[H], twiddle<T>(tw, j, sign));
-            base[0] = cmake<T>(v0.x + v1.x, v0.y + v1.y);
-            base[H] = cmake<T>(v0.x - v1.x, v0.y - v1.y);
-        }
-    }
-    __syncthreads();
-}
-
-// 16-point DFT in registers with kernel exp(sign 2 pi i r q / 16), outputs in
-// natural order: n = 4 n1 + n2, k = k1 + 4 k2 gives four 4-point DFTs over
-// n1, the twiddles exp(sign 2 pi i n2 k1 / 16), and four 4-point DFTs over n2.
-template <typename T> __device__ __forceinline__ void dft16(cplx_t<T> (&v)[16], int sign)
-{
-    const T c1 = (T)0.92387953251128675613;   // cos(pi/8)
-    const T s1 = (T)0.38268343236508977173;   // sin(pi/8)
-    const T h = (T)0.70710678118654752440;    // sqrt(1/2)
-    const T sg = (T)sign;
-    cplx_t<T> y[4][4];
-#pragma unroll
-    for (int n2 = 0; n2 < 4; ++n2) {
-        cplx_t<T> a[4] = {v[n2], v[4 + n2], v[8 + n2], v[12 + n2]};
-        dft4<T>(a, sign);
-#pragma unroll
-        for (int k1 = 0; k1 < 4; ++k1) y[n2][k1] = a[k1];
-    }
-    // z exp(sign i theta) for cos theta = c, sin theta = s
-    auto rot = [&](cplx_t<T> z, T c, T s) {
-        return cmake<T>(z.x * c - z.y * (sg * s), z.x * (sg * s) + z.y * c);
-    };
-    y[1][1] = rot(y[1][1], c1, s1);    // pi/8
-    y[1][2] = rot(y[1][2], h, h);      // pi/4
-    y[1][3] = rot(y[1][3], s1, c1);    // 3pi/8
-    y[2][1] = rot(y[2][1], h, h);      // pi/4
-    y[2][2] = cmake<T>(-sg * y[2][2].y, sg * y[2][2].x);   // pi/2
-    y[2][3] = rot(y[2][3], -h, h);     // 3pi/4
-    y[3][1] = rot(y[3][1], s1, c1);    // 3pi/8
-    y[3][2] = rot(y[3][2], -h, h);     // 3pi/4
-    y[3][3] = rot(y[3][3], -c1, -s1);  // 9pi/8
-#pragma unroll
-    for (int k1 = 0; k1 < 4; ++k1) {
-        cplx_t<T> b[4] = {y[0][k1], y[1][k1], y[2][k1], y[3][k1]};
-        dft4<T>(b, sign);
-#pragma unroll
-        for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = b[k2];
-    }
-}
-
-// One radix-16 Stockham stage (power-of-two L, Ns = 2^logNs): butterfly j of
-// line c reads j + r Q (Q = L / 16), multiplies input r by
-// exp(sign 2 pi i r (j mod Ns) / (16 Ns)), and writes its 16-point DFT to
-// (j div Ns) 16 Ns + (j mod Ns) + r Ns.  A layout flag selects, per side, the
-// lines at pitch ldsL (element i at i) or the padded lines at pitch ldsP
-// (element i at i + i / 16): the first stage (Ns = 1) writes with stride 16,
-// which the padding spreads over all LDS banks.
-template <typename T, int E, bool PIN, bool POUT>
-__device__ __forceinline__ void stage16(cplx_t<T> *buf, const cplx_t<T> *__restrict__ tw, int logL,
-                                        int C, int ldsL, int ldsP, int logNs, int sign, int tid)
-{
-    const int logQ = logL - 4;
-    const int Q = 1 << logQ;
-    const int Ns = 1 << logNs;
-    const int nb = C << logQ;
-    const int pin = PIN ? ldsP : ldsL, pout = POUT ? ldsP : ldsL;
-    constexpr int KB = (E / 16 + kFftThreads - 1) / kFftThreads;
-    cplx_t<T> v[KB][16];
-#pragma unroll
-    for (int k = 0; k < KB; ++k) {
-        const int b = tid + k * kFftThreads;
-        if (b < nb) {
-            const int c = b >> logQ, j = b & (Q - 1);
-            const cplx_t<T> *base = buf + c * pin;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int i = j + r * Q;
-                v[k][r] = base[PIN ? i + (i >> 4) : i];
-            }
-            if (Ns > 1) {
-                const int step = (j & (Ns - 1)) << (logL - 4 - logNs);
-#pragma unroll
-                for (int r = 1; r < 16; ++r) v[k][r] = cmul<T>(v[k][r], twiddle<T>(tw, r * step, sign));
-            }
-            dft16<T>(v[k], sign);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < KB; ++k) {
-        const int b = tid + k * kFftThreads;
-        if (b < nb) {
-            const int c = b >> logQ, j = b & (Q - 1);
-            const int out = ((j >> logNs) << (logNs + 4)) + (j & (Ns - 1));
-            cplx_t<T> *ob = buf + c * pout;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int i = out + r * Ns;
-                ob[POUT ? i + (i >> 4) : i] = v[k][r];
-            }
-        }
-    }
-    __syncthreads();
-}
-
-// Lines of at least 256 points run two radix-16 stages first, the first
-// writing the padded layout; LDS elements per line of the widest layout.
-__host__ __device__ constexpr bool fft_radix16(int logL) { return logL >= 8; }
-__host__ __device__ constexpr int fft_lds_pitch(int L, int logL, int ldsL)
-{
-    return fft_radix16(logL) && L + (L >> 4) > ldsL ? L + (L >> 4) : ldsL;
 }
 
 // a = q d + r for 0 <= a < 2^22 with rd = 1/d in FP32 (exact after one
@@ -371,7 +204,7 @@ __device__ __forceinline__ void fft_pass(const FftPass<T> &P, int64_t blk)
     __shared__ int s_i1[kMaxRowsPerGroup];          // SPLIT_A: index i1 of the column
 
     const int tid = threadIdx.x;
-    const int L = P.L, logL = P.logL, C = P.C, logC = P.logC, ldsL = P.ldsL;
+    const int L = P.L, C = P.C, logC = P.logC, ldsL = P.ldsL;
     const bool rows = (P.S == 1);
     int64_t pa0, s0;
     if (rows) {
@@ -400,12 +233,10 @@ __device__ __forceinline__ void fft_pass(const FftPass<T> &P, int64_t blk)
     }
     if (SPLIT == SPLIT_A && tid < C) s_i1[tid] = (int)((s0 + tid) / P.So);
     // the twiddle table of the axis, staged in LDS after the lines
-    const int ldsP = L + (L >> 4);   // padded line pitch of the radix-16 stages
-    C2 *twl = buf + C * fft_lds_pitch(L, logL, ldsL);
+    C2 *twl = buf + C * ldsL;
     for (int q = tid; q < L; q += kFftThreads) twl[q] = P.tw[q];
     __syncthreads();
 
-    const bool pow2 = logL >= 0;
     const float rL = 1.0f / (float)L;
     const int total = C * L;
     const int64_t Lf = P.Lf;
@@ -437,12 +268,7 @@ __device__ __forceinline__ void fft_pass(const FftPass<T> &P, int64_t blk)
                 const int e = e0 + u * kFftThreads;
                 int c, i;
                 if (rows) {
-                    if (pow2) {
-                        c = e >> logL;
-                        i = e & (L - 1);
-                    } else {
-                        divmod_small(e, L, rL, c, i);
-                    }
+                    divmod_small(e, L, rL, c, i);
                 } else {
                     c = e & (C - 1);
                     i = e >> logC;
@@ -492,51 +318,28 @@ __device__ __forceinline__ void fft_pass(const FftPass<T> &P, int64_t blk)
         stage_in(std::false_type{});
     __syncthreads();
 
-    if (pow2) {
-        int logNs = 0;
-        if (fft_radix16(logL)) {
-            stage16<T, E, false, true>(buf, twl, logL, C, ldsL, ldsP, 0, P.sign, tid);
-            stage16<T, E, true, false>(buf, twl, logL, C, ldsL, ldsP, 4, P.sign, tid);
-            logNs = 8;
-            while (logNs + 4 <= logL) {
-                stage16<T, E, false, false>(buf, twl, logL, C, ldsL, ldsP, logNs, P.sign, tid);
-                logNs += 4;
-            }
-        }
-        while (logNs + 2 <= logL) {
-            stage4<T, E>(buf, twl, logL, C, ldsL, logNs, P.sign, tid);
-            logNs += 2;
-        }
-        if (logNs < logL) stage2_last<T, E>(buf, twl, logL, C, ldsL, P.sign, tid);
-    } else {
-        // L = 2^a 3^b: radix 4 while the power-of-two part allows, one radix 2
-        // if a is odd, then b radix-3 stages
-        int p2 = L;
-        for (int k = 0; k < P.n3; ++k) p2 /= 3;
-        int Ns = 1;
-        while (Ns * 4 <= p2) {
-            stage_any<T, E, 4>(buf, twl, L, C, ldsL, Ns, P.sign, tid);
-            Ns *= 4;
-        }
-        if (Ns < p2) {
-            stage_any<T, E, 2>(buf, twl, L, C, ldsL, Ns, P.sign, tid);
-            Ns *= 2;
-        }
-        for (int k = 0; k < P.n3; ++k) {
-            stage_any<T, E, 3>(buf, twl, L, C, ldsL, Ns, P.sign, tid);
-            Ns *= 3;
-        }
+    // L = 2^a 3^b: radix 4 while the power-of-two part allows, one radix 2 if a
+    // is odd, then b radix-3 stages
+    int p2 = L;
+    for (int k = 0; k < P.n3; ++k) p2 /= 3;
+    int Ns = 1;
+    while (Ns * 4 <= p2) {
+        stage_any<T, E, 4>(buf, twl, L, C, ldsL, Ns, P.sign, tid);
+        Ns *= 4;
+    }
+    if (Ns < p2) {
+        stage_any<T, E, 2>(buf, twl, L, C, ldsL, Ns, P.sign, tid);
+        Ns *= 2;
+    }
+    for (int k = 0; k < P.n3; ++k) {
+        stage_any<T, E, 3>(buf, twl, L, C, ldsL, Ns, P.sign, tid);
+        Ns *= 3;
     }
 
     for (int e = tid; e < total; e += kFftThreads) {
         int c, i;
         if (rows) {
-            if (pow2) {
-                c = e >> logL;
-                i = e & (L - 1);
-            } else {
-                divmod_small(e, L, rL, c, i);
-            }
+            divmod_small(e, L, rL, c, i);
         } else {
             c = e & (C - 1);
             i = e >> logC;
@@ -590,26 +393,25 @@ void launch_fft_pass(const FftPass<T> &p, int64_t blocks, size_t lds_bytes, hipS
     if (blocks <= 0) return;
     if (blocks >= (int64_t(1) << 32) / kFftThreads)
         throw Error(CUNFFT_ERR_UNSUPPORTED, "FFT pass needs too many workgroups");
-    static_assert(fft_max_elems<float>() == kFftSmallElems && fft_max_elems<double>() == kFftSmallElems,
-                  "one LDS line size");
+    if (p.tpl > 0) {
+        launch_fft_line<T>(p, blocks, lds_bytes, s);
+        return;
+    }
     if (p.split == SPLIT_A)
-        k_fft_pass<T, kFftSmallElems, SPLIT_A><<<(unsigned)blocks, kFftThreads, lds_bytes, s>>>(p);
+        k_fft_pass<T, kFftElems, SPLIT_A><<<(unsigned)blocks, kFftThreads, lds_bytes, s>>>(p);
     else if (p.split == SPLIT_B)
-        k_fft_pass<T, kFftSmallElems, SPLIT_B><<<(unsigned)blocks, kFftThreads, lds_bytes, s>>>(p);
+        k_fft_pass<T, kFftElems, SPLIT_B><<<(unsigned)blocks, kFftThreads, lds_bytes, s>>>(p);
     else
-        k_fft_pass<T, kFftSmallElems, SPLIT_NONE><<<(unsigned)blocks, kFftThreads, lds_bytes, s>>>(p);
+        k_fft_pass<T, kFftElems, SPLIT_NONE><<<(unsigned)blocks, kFftThreads, lds_bytes, s>>>(p);
     CUNFFT_HIP(hipGetLastError());
 }
 
 template <typename T>
 void launch_fft_batch(const FftPass<T> *passes, const BlockMap *map, uint32_t nblk,
-                      size_t lds_bytes, int max_elems, hipStream_t s)
+                      size_t lds_bytes, hipStream_t s)
 {
     if (nblk == 0) return;
-    if (max_elems > kFftSmallElems)
-        k_fft_pass_batch<T, fft_max_elems<T>()><<<nblk, kFftThreads, lds_bytes, s>>>(passes, map);
-    else
-        k_fft_pass_batch<T, kFftSmallElems><<<nblk, kFftThreads, lds_bytes, s>>>(passes, map);
+    k_fft_pass_batch<T, kFftElems><<<nblk, kFftThreads, lds_bytes, s>>>(passes, map);
     CUNFFT_HIP(hipGetLastError());
 }
 
@@ -634,19 +436,83 @@ static int64_t next_pow2_i(int64_t v)
     return p;
 }
 
-// Lines per workgroup: rows (S = 1) are packed up to 2048 elements per
-// workgroup; strided passes take C adjacent columns (coalesced C-wide reads)
-// up to 4096 elements.  Sets C, logC, ldsL and the launch's blocks and LDS
-// from P.L, P.S and P.n_pa.
-template <typename T> static void pass_shape(FftLaunch<T> &out)
+// Threads per line of the register-resident pass for P, or 0: its line length
+// is not listed, or its counts leave 32 bits.
+template <typename T> static int line_tpl(const FftPass<T> &P)
+{
+    int64_t total = P.Lf * P.So;
+    for (int q = 0; q < P.t; ++q) total *= P.n[q];
+    if (total >= (int64_t(1) << 32) || P.n_pa >= (int64_t(1) << 31) || P.S >= (int64_t(1) << 31)) return 0;
+    switch (P.L) {
+#define CUNFFT_CASE(LEN) \
+    case LEN: return LEN / LinePlan<LEN>::EPT;
+        CUNFFT_POW2_LINES(CUNFFT_CASE)
+        CUNFFT_MIXED_LINES(CUNFFT_CASE)
+#undef CUNFFT_CASE
+    }
+    return 0;
+}
+template <typename T> static bool line_split_ok(const FftPass<T> &P)
+{
+    switch (P.L) {
+#define CUNFFT_CASE(LEN) case LEN:
+        CUNFFT_SPLIT_LINES(CUNFFT_CASE)
+#undef CUNFFT_CASE
+        return true;
+    }
+    return false;
+}
+static int line_pitch_of(int L)
+{
+    switch (L) {
+#define CUNFFT_CASE(LEN) \
+    case LEN: return line_pitch<LEN>();
+        CUNFFT_POW2_LINES(CUNFFT_CASE)
+        CUNFFT_MIXED_LINES(CUNFFT_CASE)
+#undef CUNFFT_CASE
+    }
+    return L;
+}
+
+// Lines per workgroup (C, a power of two) with the launch's blocks and LDS, from
+// P.L, P.S and P.n_pa.
+//
+// Register-resident pass: as many lines as fill 256 threads (512 from 1024
+// points on, where 256 threads hold too few adjacent columns), columns at most
+// one 128-byte line wide.  A small grid takes fewer lines per workgroup, down to
+// one wavefront (rows) or 64 bytes of a row (columns), until 512 workgroups
+// spread over the 256 CUs.  A batch launches 256-thread workgroups for all its
+// jobs, which are many: always full ones.
+//
+// Generic pass: rows are packed up to 2048 elements per workgroup; strided
+// passes take adjacent columns up to kFftElems elements.
+template <typename T> static void pass_shape(FftLaunch<T> &out, FftUse use)
 {
     FftPass<T> &P = out.P;
-    P.logL = (P.L & (P.L - 1)) == 0 ? ilog2_i(P.L) : -1;
     P.n3 = 0;
     for (int l = P.L; l % 3 == 0; l /= 3) ++P.n3;
-    const int64_t target = 2048;
+    P.tpl = line_tpl<T>(P);
+    if (P.split != SPLIT_NONE && !line_split_ok<T>(P)) P.tpl = 0;
+    if (use == FFT_GRADIENT && sizeof(T) == 4 && P.n3 > 0) P.tpl = 0;
+    const bool batch = use == FFT_BATCH;
     int64_t C;
-    if (P.S == 1) {
+    if (P.tpl > 0) {
+        constexpr int cs = (int)sizeof(cplx_t<T>);
+        const int64_t most = batch || P.L < 1024 ? 256 : 512;
+        const int64_t wide = P.split == SPLIT_B && P.S == 1 ? P.L2 & -P.L2 : P.S & -P.S;
+        const size_t line = (size_t)line_pitch_of(P.L) * cs;
+        const bool rows = P.S == 1, side = !rows || P.split == SPLIT_B;   // side by side in memory
+        C = std::max<int64_t>(1, prev_pow2_i(most / P.tpl));
+        if (side) C = std::min<int64_t>(std::min<int64_t>(C, 128 / cs), wide);
+        else C = std::min<int64_t>(C, next_pow2_i(P.n_pa));
+        while (C > 1 && C * line > (size_t)kFftLineLds) C >>= 1;
+        auto blocks = [&](int64_t c) { return rows ? (P.n_pa + c - 1) / c : P.n_pa * (P.S / c); };
+        while (!batch && C > 1 && blocks(C) < 512 && (side ? C * cs > 64 : C * P.tpl > 64)) C >>= 1;
+        out.blocks = blocks(C);
+        P.ldsL = 0;
+        out.lds = (size_t)C * line;
+    } else if (P.S == 1) {
+        const int64_t target = 2048;
         C = P.L >= target ? 1 : prev_pow2_i(target / P.L);
         C = std::min<int64_t>(C, 64);
         C = std::min<int64_t>(C, next_pow2_i(P.n_pa));
@@ -656,14 +522,14 @@ template <typename T> static void pass_shape(FftLaunch<T> &out)
         // adjacent columns: C divides S (the largest power of two in S bounds it)
         const int64_t cdef = sizeof(T) == 8 ? 8 : 16;
         C = std::min<int64_t>(cdef, P.S & -P.S);
-        C = std::min<int64_t>(C, std::max<int64_t>(1, prev_pow2_i(fft_max_elems<T>() / P.L)));
+        C = std::min<int64_t>(C, std::max<int64_t>(1, prev_pow2_i(kFftElems / P.L)));
         out.blocks = P.n_pa * (P.S / C);
         P.ldsL = C > 1 ? P.L + 1 : P.L;
     }
     P.C = (int)C;
     P.logC = ilog2_i(C);
-    // lines (at the widest pitch the stages use) + twiddles
-    out.lds = ((size_t)C * fft_lds_pitch(P.L, P.logL, P.ldsL) + P.L) * sizeof(cplx_t<T>);
+    // generic pass: lines + twiddles
+    if (P.tpl == 0) out.lds = ((size_t)C * P.ldsL + P.L) * sizeof(cplx_t<T>);
 }
 
 template <typename T>
@@ -697,7 +563,7 @@ static FftPass<T> pass_common(const Geom &ge, const double *roc, const int64_t *
 template <typename T>
 FftLaunch<T> fft_pass_setup(const Geom &ge, const cplx_t<T> *tw, const double *roc,
                             const int64_t *rocoff, int t, bool forward, const cplx_t<T> *fhat_in,
-                            cplx_t<T> *fhat_out, cplx_t<T> *g)
+                            cplx_t<T> *fhat_out, cplx_t<T> *g, FftUse use)
 {
     const int d = ge.d;
     FftLaunch<T> out{};
@@ -712,18 +578,18 @@ FftLaunch<T> fft_pass_setup(const Geom &ge, const cplx_t<T> *tw, const double *r
         P.mode = (t == d - 1) ? FFT_FROM_FHAT : FFT_IN_PRUNED;
     else
         P.mode = (t == d - 1) ? FFT_TO_FHAT : FFT_OUT_PRUNED;
-    pass_shape<T>(out);
+    pass_shape<T>(out, use);
     return out;
 }
 
 template <typename T>
 int fft_axis_setup(const Geom &ge, const cplx_t<T> *const *tw, const double *roc,
                    const int64_t *rocoff, int t, bool forward, const cplx_t<T> *fhat_in,
-                   cplx_t<T> *fhat_out, cplx_t<T> **g, cplx_t<T> **g_other, FftLaunch<T> *out)
+                   cplx_t<T> *fhat_out, cplx_t<T> **g, cplx_t<T> **g_other, FftLaunch<T> *out, FftUse use)
 {
     const int d = ge.d;
     if (fft_line_ok(ge.n[t])) {
-        out[0] = fft_pass_setup<T>(ge, tw[0], roc, rocoff, t, forward, fhat_in, fhat_out, *g);
+        out[0] = fft_pass_setup<T>(ge, tw[0], roc, rocoff, t, forward, fhat_in, fhat_out, *g, use);
         return 1;
     }
     int64_t L1, L2;
@@ -740,7 +606,7 @@ int fft_axis_setup(const Geom &ge, const cplx_t<T> *const *tw, const double *roc
     A.P.L1 = L1;
     A.P.L2 = L2;
     A.P.mode = forward ? ((t == d - 1) ? FFT_FROM_FHAT : FFT_IN_PRUNED) : 0;
-    pass_shape<T>(A);
+    pass_shape<T>(A, use);
     // B: per k2 the L1-point FFT over i1 with the w_Lf twiddles, to the other
     // grid in natural order (or to fhat with the crop and roll-off)
     FftLaunch<T> &B = out[1];
@@ -754,7 +620,7 @@ int fft_axis_setup(const Geom &ge, const cplx_t<T> *const *tw, const double *roc
     B.P.n_pa *= L2;
     B.P.mode = forward ? 0 : ((t == d - 1) ? FFT_TO_FHAT : FFT_OUT_PRUNED);
     B.P.dst = B.P.mode == FFT_TO_FHAT ? nullptr : *g_other;
-    pass_shape<T>(B);
+    pass_shape<T>(B, use);
     if (B.P.mode != FFT_TO_FHAT) std::swap(*g, *g_other);
     return 2;
 }
@@ -762,20 +628,20 @@ int fft_axis_setup(const Geom &ge, const cplx_t<T> *const *tw, const double *roc
 template void launch_fft_pass<float>(const FftPass<float> &, int64_t, size_t, hipStream_t);
 template void launch_fft_pass<double>(const FftPass<double> &, int64_t, size_t, hipStream_t);
 template void launch_fft_batch<float>(const FftPass<float> *, const BlockMap *, uint32_t, size_t,
-                                      int, hipStream_t);
+                                      hipStream_t);
 template void launch_fft_batch<double>(const FftPass<double> *, const BlockMap *, uint32_t, size_t,
-                                       int, hipStream_t);
+                                       hipStream_t);
 template FftLaunch<float> fft_pass_setup<float>(const Geom &, const float2 *, const double *,
                                                 const int64_t *, int, bool, const float2 *,
-                                                float2 *, float2 *);
+                                                float2 *, float2 *, FftUse);
 template FftLaunch<double> fft_pass_setup<double>(const Geom &, const double2 *, const double *,
                                                   const int64_t *, int, bool, const double2 *,
-                                                  double2 *, double2 *);
+                                                  double2 *, double2 *, FftUse);
 template int fft_axis_setup<float>(const Geom &, const float2 *const *, const double *,
                                    const int64_t *, int, bool, const float2 *, float2 *, float2 **,
-                                   float2 **, FftLaunch<float> *);
+                                   float2 **, FftLaunch<float> *, FftUse);
 template int fft_axis_setup<double>(const Geom &, const double2 *const *, const double *,
                                     const int64_t *, int, bool, const double2 *, double2 *,
-                                    double2 **, double2 **, FftLaunch<double> *);
+                                    double2 **, double2 **, FftLaunch<double> *, FftUse);
 
 }  // namespace cunfft

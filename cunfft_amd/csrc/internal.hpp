@@ -108,12 +108,13 @@ template <typename T> struct FftPass {
     int64_t n[3];
     int64_t N[3];
     int d, t;
-    int L, logL;             // logL = log2(L) for a power of two, else -1
+    int L;
     int n3;                  // radix-3 factors of L (L = 2^a 3^n3)
+    int tpl;                 // threads per line of the register-resident pass; 0: the generic pass
     int64_t S;
     int64_t n_pa;            // number of lines over the axes before t (times L2 for SPLIT_B)
     int C, logC;             // lines per workgroup
-    int ldsL;                // LDS row pitch in elements
+    int ldsL;                // LDS row pitch in elements (generic pass)
     int sign;                // -1 forward, +1 adjoint
     int mode;
     // split axes
@@ -126,11 +127,20 @@ template <typename T> struct FftPass {
 
 template <typename T>
 void launch_fft_pass(const FftPass<T> &p, int64_t blocks, size_t lds_bytes, hipStream_t s);
+// The register-resident form (fft_line.hpp; passes with tpl > 0).
+template <typename T>
+void launch_fft_line(const FftPass<T> &p, int64_t blocks, size_t lds_bytes, hipStream_t s);
 
 // Pass along axis t of one transform (forward: axes d-1 .. 0, the first from
 // fhat with the roll-off; adjoint: axes 0 .. d-1, the last to fhat), with its
 // launch shape.  tw is the twiddle table of length n_t.  Axes longer than
 // kFftMaxLine need fft_axis_setup.
+// What a pass is set up for: a transform of its own, a batch's launch over many
+// (256-thread workgroups), or the grid of an FP32 node gradient.  The gradient is
+// handed out as float64 values (autograd.py), so its bits are kept: the mixed
+// line lengths, whose radices the register-resident pass orders differently, run
+// the generic pass there (the power-of-two lines give the same bits in both).
+enum FftUse : int { FFT_SINGLE = 0, FFT_BATCH, FFT_GRADIENT };
 template <typename T> struct FftLaunch {
     FftPass<T> P;
     int64_t blocks;
@@ -139,7 +149,7 @@ template <typename T> struct FftLaunch {
 template <typename T>
 FftLaunch<T> fft_pass_setup(const Geom &ge, const cplx_t<T> *tw, const double *roc,
                             const int64_t *rocoff, int t, bool forward, const cplx_t<T> *fhat_in,
-                            cplx_t<T> *fhat_out, cplx_t<T> *g);
+                            cplx_t<T> *fhat_out, cplx_t<T> *g, FftUse use = FFT_SINGLE);
 // The passes of axis t (one, or two for a split axis): tw[0] is the twiddle
 // table of the axis (n_t), or of L1 and tw[1] of L2 when it is split.  The
 // axis's data is in *g; a split axis leaves it in g_other and swaps the two
@@ -147,18 +157,23 @@ FftLaunch<T> fft_pass_setup(const Geom &ge, const cplx_t<T> *tw, const double *r
 template <typename T>
 int fft_axis_setup(const Geom &ge, const cplx_t<T> *const *tw, const double *roc,
                    const int64_t *rocoff, int t, bool forward, const cplx_t<T> *fhat_in,
-                   cplx_t<T> *fhat_out, cplx_t<T> **g, cplx_t<T> **g_other, FftLaunch<T> *out);
+                   cplx_t<T> *fhat_out, cplx_t<T> **g, cplx_t<T> **g_other, FftLaunch<T> *out,
+                   FftUse use = FFT_SINGLE);
 
 // Workgroup b of a batched launch works on block map[b].blk of job map[b].job.
 struct BlockMap {
     uint32_t job;
     uint32_t blk;
 };
-// One launch of the passes of many transforms (one FftPass per job);
-// max_elems = the largest C * L of the passes.
+// One launch of the passes of many transforms (one FftPass per job): generic
+// passes, or register-resident ones set up for a batch (rows: along the last
+// axis).
 template <typename T>
 void launch_fft_batch(const FftPass<T> *passes, const BlockMap *map, uint32_t nblk,
-                      size_t lds_bytes, int max_elems, hipStream_t s);
+                      size_t lds_bytes, hipStream_t s);
+template <typename T>
+void launch_fft_line_batch(const FftPass<T> *passes, const BlockMap *map, uint32_t nblk, bool rows,
+                           size_t lds_bytes, hipStream_t s);
 
 // ------------------------------------------------------------ gridding ---
 template <typename T>

@@ -498,7 +498,7 @@ template <typename T> static void finalize(typename Traits<T>::plan *p)
 template <typename T>
 static cplx_t<T> *fft_passes(typename Traits<T>::plan *p, Impl<T> *im, FftTables *ft, bool forward,
                              const cplx_t<T> *fhat_in, cplx_t<T> *fhat_out, cplx_t<T> *g,
-                             hipStream_t s)
+                             hipStream_t s, FftUse use = FFT_SINGLE)
 {
     const int d = p->d;
     cplx_t<T> *cur = g;
@@ -509,7 +509,7 @@ static cplx_t<T> *fft_passes(typename Traits<T>::plan *p, Impl<T> *im, FftTables
                                   static_cast<const cplx_t<T> *>(ft->tw2[t])};
         FftLaunch<T> L[2];
         const int np = fft_axis_setup<T>(im->geom, tw, im->roc, im->rocoff, t, forward, fhat_in,
-                                         fhat_out, &cur, &other, L);
+                                         fhat_out, &cur, &other, L, use);
         for (int i = 0; i < np; ++i) launch_fft_pass<T>(L[i].P, L[i].blocks, L[i].lds, s);
     }
     im->g_last = cur;
@@ -1066,7 +1066,7 @@ int api_grad_x_dev(typename Traits<T>::plan *p, const void *fhat, const void *v,
         hipStream_t s = pick_stream(stream, im->stream);
         const cplx_t<T> *g = fft_passes<T>(p, im, fft_tables<T>(p, true), true,
                                            static_cast<const cplx_t<T> *>(fhat), nullptr,
-                                           reinterpret_cast<cplx_t<T> *>(p->g_gpu), s);
+                                           reinterpret_cast<cplx_t<T> *>(p->g_gpu), s, FFT_GRADIENT);
         grad_x<T>(p, im, g, static_cast<const cplx_t<T> *>(v), gx, s);
     });
 }
@@ -1089,7 +1089,7 @@ int api_backward_dev(typename Traits<T>::plan *p, const void *fhat, const void *
         if (gx) {
             const cplx_t<T> *g = fft_passes<T>(p, im, fft_tables<T>(p, true), true,
                                                static_cast<const cplx_t<T> *>(fhat), nullptr,
-                                               reinterpret_cast<cplx_t<T> *>(p->g_gpu), s);
+                                               reinterpret_cast<cplx_t<T> *>(p->g_gpu), s, FFT_GRADIENT);
             grad_x<T>(p, im, g, static_cast<const cplx_t<T> *>(gf), gx, s);
         }
         if (gfhat) {

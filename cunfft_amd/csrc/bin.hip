@@ -1,14 +1,13 @@
-// bin.hip -- node binning and the node-per-lane tiled gridding kernels.
+// bin.hip -- the node-per-lane tiled gridding kernels.
 //
 // The reference grids one node per thread straight from global memory: the
 // forward through a texture copy of the grid (src/cunfft_kernel.cu:514-1093,
 // 1408-1418), the adjoint with two CAS-loop atomics per tap into global memory
-// (src/cunfft_kernel.cu:97-130, 608-1197).  Here nodes are first sorted on the
-// device by the grid tile holding their window start (a stable radix sort of
-// composite keys, then tile counts, scans and chunks), and each workgroup then
+// (src/cunfft_kernel.cu:97-130, 608-1197).  Here nodes are first sorted by the
+// grid tile holding their window start (binning.hip), and each workgroup then
 // owns one tile.  For d >= 2 the plane-tiled kernels of grid_tile.hpp use the
-// sorted order; this file holds the binning itself and the node-per-lane
-// tiled kernels used for d = 1 and under CUNFFT_NODE_LANES:
+// sorted order; this file holds the node-per-lane tiled kernels used for d = 1
+// and under CUNFFT_NODE_LANES:
 //   forward  the padded tile (T_t + 2m + 1 cells per axis) is staged in LDS
 //            once, and every node of the tile reads its (2m+2)^d taps there;
 //   adjoint  the node contributions accumulate in an LDS copy of the padded
@@ -38,535 +37,6 @@ template <int D, int W> struct Pad {
 template <typename T, int D, int W> constexpr bool tile_fits()
 {
     return (size_t)Pad<D, W>::PT * 2 * sizeof(T) <= (size_t)kMaxTileBytes;
-}
-
-BinGeom bin_geom(const Binning &b)
-{
-    BinGeom g{};
-    g.d = b.d;
-    for (int t = 0; t < 3; ++t) {
-        int l = 0;
-        while ((int64_t(1) << l) < b.T[t]) ++l;
-        g.logT[t] = l;
-        g.nt[t] = b.nt[t];
-    }
-    g.ntiles = b.ntiles;
-    g.sub_shift = b.elem_bytes == 4 ? 1 : 0;
-    return g;
-}
-
-// ----------------------------------------------------------- binning ----
-__global__ __launch_bounds__(256) void k_fill_u32(uint32_t *p, int64_t n, uint32_t v)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-// Composite sort key of every node (its tile times sub_range plus, for the
-// plane-tiled kernels, its sub_key within the tile; sub_range 1 otherwise)
-// and (plane-tiled kernels) its window descriptor by node index: the FP64
-// index/fraction split of window_cell, lo_t the window start relative to the
-// origin of the node's tile, in [0, T_t) by construction of the key.  The
-// tile counts come from the sorted keys (k_bin_tile_first / _count), not from
-// atomics here: a node cluster would serialize them on a few counters.
-template <typename T>
-__global__ __launch_bounds__(256) void k_bin_keys(const double *__restrict__ x,
-                                                  uint32_t *__restrict__ keys,
-                                                  NodeDesc<T> *__restrict__ desc_j, Geom ge,
-                                                  BinGeom bg, uint32_t sub_range)
-{
-    const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (j >= ge.M) return;
-    uint32_t tile = 0, loc = 0;
-    uint32_t lo[3] = {0, 0, 0};
-    NodeDesc<T> nd{};
-    for (int t = 0; t < bg.d; ++t) {
-        double c;
-        const int64_t w = window_cell(x[j * bg.d + t], ge.n[t], ge.m, c);
-        const uint32_t tc = (uint32_t)(w >> bg.logT[t]);
-        lo[t] = (uint32_t)(w - ((int64_t)tc << bg.logT[t]));
-        loc |= lo[t] << (8 * t);
-        nd.f[t] = (T)(c - (double)ge.m);
-        tile = tile * (uint32_t)bg.nt[t] + tc;
-    }
-    keys[j] = sub_range > 1 ? tile * sub_range + sub_key(bg.d, lo, bg.logT, bg.sub_shift) : tile;
-    if (desc_j) {
-        nd.loc = loc;
-        desc_j[j] = nd;
-    }
-}
-
-// First sorted position of every nonempty tile, from the sorted composite keys.
-__global__ __launch_bounds__(256) void k_bin_tile_first(const uint32_t *__restrict__ skeys, int64_t M,
-                                                        uint32_t sub_range, uint32_t *__restrict__ first)
-{
-    const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (s >= M) return;
-    const uint32_t t = skeys[s] / sub_range;
-    if (s == 0 || skeys[s - 1] / sub_range != t) first[t] = (uint32_t)s;
-}
-
-// Node count of every nonempty tile, written at its last sorted position
-// (empty tiles keep the zero they were filled with).
-__global__ __launch_bounds__(256) void k_bin_tile_count(const uint32_t *__restrict__ skeys, int64_t M,
-                                                        uint32_t sub_range,
-                                                        const uint32_t *__restrict__ first,
-                                                        uint32_t *__restrict__ cnt)
-{
-    const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (s >= M) return;
-    const uint32_t t = skeys[s] / sub_range;
-    if (s == M - 1 || skeys[s + 1] / sub_range != t) cnt[t] = (uint32_t)s + 1u - first[t];
-}
-
-// Exclusive scans of the tile counts and of the chunk counts, in three
-// launches: sums per block of kScanBlock tiles, one workgroup scanning those
-// sums, then each block's own scan plus its offset.
-constexpr int kScanBlock = 1024;
-
-// Inclusive scan of (a, b) over a workgroup of kScanBlock threads: wavefront
-// scans with shuffles, then the wavefront totals through LDS.
-__device__ __forceinline__ void block_scan2(uint32_t &a, uint32_t &b, uint32_t *wa, uint32_t *wb)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t va = __shfl_up(a, off, 64), vb = __shfl_up(b, off, 64);
-        if (lane >= off) {
-            a += va;
-            b += vb;
-        }
-    }
-    if (lane == 63) {
-        wa[wave] = a;
-        wb[wave] = b;
-    }
-    __syncthreads();
-    if (wave == 0) {
-        uint32_t ta = lane < kScanBlock / 64 ? wa[lane] : 0u, tb = lane < kScanBlock / 64 ? wb[lane] : 0u;
-        for (int off = 1; off < kScanBlock / 64; off <<= 1) {
-            const uint32_t va = __shfl_up(ta, off, 64), vb = __shfl_up(tb, off, 64);
-            if (lane >= off) {
-                ta += va;
-                tb += vb;
-            }
-        }
-        if (lane < kScanBlock / 64) {
-            wa[lane] = ta;
-            wb[lane] = tb;
-        }
-    }
-    __syncthreads();
-    if (wave > 0) {
-        a += wa[wave - 1];
-        b += wb[wave - 1];
-    }
-}
-
-// (a, b) = (count, chunks of count) of element i of cnt, or of the digit
-// counts when chunks is false (b then unused).
-__global__ __launch_bounds__(kScanBlock) void k_bin_scan_part(const uint32_t *__restrict__ cnt,
-                                                              uint32_t *__restrict__ part,
-                                                              int64_t ntiles, int64_t nparts)
-{
-    __shared__ uint32_t wa[kScanBlock / 64], wb[kScanBlock / 64];
-    const int64_t i = (int64_t)blockIdx.x * kScanBlock + threadIdx.x;
-    const uint32_t c = i < ntiles ? cnt[i] : 0u;
-    uint32_t a = c, b = (c + kChunk - 1) / kChunk;
-    block_scan2(a, b, wa, wb);
-    if (threadIdx.x == kScanBlock - 1) {
-        part[blockIdx.x] = a;
-        part[nparts + blockIdx.x] = b;
-    }
-}
-
-// One workgroup: exclusive scan of the block sums in place; the chunk total
-// (n_chunks may be NULL).
-__global__ __launch_bounds__(kScanBlock) void k_bin_scan_top(uint32_t *__restrict__ part,
-                                                             int64_t nparts,
-                                                             uint32_t *__restrict__ n_chunks)
-{
-    __shared__ uint32_t wa[kScanBlock / 64], wb[kScanBlock / 64];
-    uint32_t ca = 0, cb = 0;
-    for (int64_t base = 0; base < nparts; base += kScanBlock) {
-        const int64_t i = base + threadIdx.x;
-        const uint32_t a0 = i < nparts ? part[i] : 0u, b0 = i < nparts ? part[nparts + i] : 0u;
-        uint32_t a = a0, b = b0;
-        block_scan2(a, b, wa, wb);
-        if (i < nparts) {
-            part[i] = ca + a - a0;
-            part[nparts + i] = cb + b - b0;
-        }
-        __syncthreads();   // every thread has its block totals before wa/wb are reused
-        ca += wa[kScanBlock / 64 - 1];
-        cb += wb[kScanBlock / 64 - 1];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && n_chunks) n_chunks[0] = cb;
-}
-
-// start = exclusive scan of cnt; chunk_start (may be NULL) = exclusive scan
-// of the chunk counts.  start may be cnt itself (in place).
-__global__ __launch_bounds__(kScanBlock) void k_bin_scan_apply(const uint32_t *cnt,
-                                                               const uint32_t *__restrict__ part,
-                                                               uint32_t *start,
-                                                               uint32_t *__restrict__ chunk_start,
-                                                               int64_t ntiles, int64_t nparts)
-{
-    __shared__ uint32_t wa[kScanBlock / 64], wb[kScanBlock / 64];
-    const int64_t i = (int64_t)blockIdx.x * kScanBlock + threadIdx.x;
-    const uint32_t c = i < ntiles ? cnt[i] : 0u, cc = (c + kChunk - 1) / kChunk;
-    uint32_t a = c, b = cc;
-    block_scan2(a, b, wa, wb);
-    if (i < ntiles) {
-        start[i] = part[blockIdx.x] + a - c;
-        if (chunk_start) chunk_start[i] = part[nparts + blockIdx.x] + b - cc;
-    }
-}
-
-// ------------------------------------------------------- radix sort ----
-// Stable LSD radix sort of (composite key, node index) pairs, 8-bit digits.
-// Each pass: per-block digit counts (k_rs_hist), an exclusive scan of the
-// counts in digit-major order (digit d of block b at d * nblk + b), then a
-// stable scatter (k_rs_scatter) in which block b walks its items in order,
-// 256 at a time, and ranks each among the earlier items of its digit: within
-// a wavefront from ballots on the digit's bits, across the block's wavefronts
-// and rounds from LDS counters.  No atomic decides a position, so the result
-// is the same on every run.
-constexpr int kRsThreads = 256;
-constexpr int kRsRounds = 16;
-constexpr int kRsItems = kRsThreads * kRsRounds;   // items per block
-constexpr int kRsDigits = 256;
-
-__global__ __launch_bounds__(kRsThreads) void k_rs_hist(const uint32_t *__restrict__ keys, int64_t M,
-                                                        int shift, uint32_t *__restrict__ hist,
-                                                        uint32_t nblk)
-{
-    __shared__ uint32_t h[kRsDigits];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t i0 = (int64_t)blockIdx.x * kRsItems + threadIdx.x;
-#pragma unroll 4
-    for (int k = 0; k < kRsRounds; ++k) {
-        const int64_t i = i0 + (int64_t)k * kRsThreads;
-        if (i < M) atomicAdd(&h[(keys[i] >> shift) & 255u], 1u);
-    }
-    __syncthreads();
-    hist[(size_t)threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
-}
-
-// vals_in NULL: the values are the item indices (the first pass over node
-// order).  keys_out may be NULL when the sorted keys are not needed.
-__global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const uint32_t *__restrict__ keys_in,
-                                                           const uint32_t *__restrict__ vals_in,
-                                                           int64_t M, int shift,
-                                                           const uint32_t *__restrict__ offs,
-                                                           uint32_t nblk,
-                                                           uint32_t *__restrict__ keys_out,
-                                                           uint32_t *__restrict__ vals_out)
-{
-    __shared__ uint32_t base[kRsDigits];                        // next position per digit
-    __shared__ uint32_t wcnt[kRsThreads / 64][kRsDigits];       // this digit pass's count per wavefront
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    base[tid] = offs[(size_t)tid * nblk + blockIdx.x];
-#pragma unroll
-    for (int w = 0; w < kRsThreads / 64; ++w) wcnt[w][tid] = 0;
-    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    __syncthreads();
-    const int64_t i0 = (int64_t)blockIdx.x * kRsItems + tid;
-    for (int k = 0; k < kRsRounds; ++k) {
-        const int64_t i = i0 + (int64_t)k * kRsThreads;
-        if (((int64_t)blockIdx.x * kRsItems + (int64_t)k * kRsThreads) >= M) break;   // uniform
-        const bool valid = i < M;
-        const uint32_t key = valid ? keys_in[i] : 0u;
-        const uint32_t val = valid ? (vals_in ? vals_in[i] : (uint32_t)i) : 0u;
-        const uint32_t dg = (key >> shift) & 255u;
-        // lanes of this wavefront holding the same digit (valid lanes only)
-        uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int bit = 0; bit < 8; ++bit) {
-            const uint64_t ones = __ballot(valid && ((dg >> bit) & 1u));
-            peers &= ((dg >> bit) & 1u) ? ones : ~ones;
-        }
-        const uint32_t rank = (uint32_t)__popcll(peers & below);
-        if (valid && rank == 0) wcnt[wave][dg] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        if (valid) {
-            uint32_t pos = base[dg] + rank;
-            for (int w = 0; w < wave; ++w) pos += wcnt[w][dg];
-            if (keys_out) keys_out[pos] = key;
-            vals_out[pos] = val;
-        }
-        __syncthreads();
-        uint32_t tot = 0;
-#pragma unroll
-        for (int w = 0; w < kRsThreads / 64; ++w) {
-            tot += wcnt[w][tid];
-            wcnt[w][tid] = 0;
-        }
-        base[tid] += tot;
-        __syncthreads();
-    }
-}
-
-// Sorted-order copies of the per-node data: descriptors (plane-tiled
-// kernels) or coordinates (node-lane kernels).
-template <typename T>
-__global__ __launch_bounds__(256) void k_bin_gather_desc(const uint32_t *__restrict__ perm,
-                                                         const NodeDesc<T> *__restrict__ desc_j,
-                                                         NodeDesc<T> *__restrict__ desc, int64_t M)
-{
-    const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (s < M) desc[s] = desc_j[perm[s]];
-}
-
-__global__ __launch_bounds__(256) void k_bin_gather_x(const uint32_t *__restrict__ perm,
-                                                      const double *__restrict__ x,
-                                                      double *__restrict__ xs, int64_t M, int d)
-{
-    const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (s >= M) return;
-    const int64_t j = perm[s];
-    for (int t = 0; t < d; ++t) xs[s * d + t] = x[j * d + t];
-}
-
-__global__ __launch_bounds__(256) void k_bin_chunks(const uint32_t *__restrict__ cnt,
-                                                    const uint32_t *__restrict__ start,
-                                                    const uint32_t *__restrict__ chunk_start,
-                                                    Chunk *__restrict__ chunks, int64_t ntiles)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= ntiles) return;
-    const uint32_t c = cnt[i];
-    uint32_t o = chunk_start[i];
-    for (uint32_t s = 0; s < c; s += kChunk, ++o) {
-        Chunk ch;
-        ch.tile = (uint32_t)i;
-        ch.start = start[i] + s;
-        ch.count = c - s < (uint32_t)kChunk ? c - s : (uint32_t)kChunk;
-        ch.pad = 0;
-        chunks[o] = ch;
-    }
-}
-
-bool Binning::plan(const Geom &ge, int elem_bytes_, int kernel_variant, int tile_variant_)
-{
-    variant = kernel_variant;
-    tile_variant = tile_variant_;
-    elem_bytes = elem_bytes_;
-    d = ge.d;
-    usable = 0;
-    const int W = ge.W;
-    if (W > 18 || ge.M >= (int64_t(1) << 31)) return false;
-    int64_t shape[3];
-    tile_shape(d, planes() ? tile_variant : 0, shape);
-    int64_t bytes = 2 * elem_bytes;
-    ntiles = 1;
-    int64_t ncells = 1;
-    for (int t = 0; t < 3; ++t) {
-        T[t] = t < d ? shape[t] : 1;
-        if (t < d && (ge.n[t] < T[t] || ge.n[t] % T[t] != 0)) return false;
-        nt[t] = t < d ? ge.n[t] / T[t] : 1;
-        ntiles *= nt[t];
-        ncells *= t < d ? ge.n[t] : 1;
-        if (t < d) bytes *= T[t] + W - 1;
-    }
-    if (ntiles >= (int64_t(1) << 31)) return false;
-    if (planes()) {
-        // plane-tiled kernels: 32-bit grid offsets and the LDS tile must fit
-        if (ncells > (int64_t(1) << 32)) return false;
-        const bool fits = elem_bytes == 4 ? tile_kernels_fit<float>(ge, tile_variant, compensated)
-                                          : tile_kernels_fit<double>(ge, tile_variant, false);
-        if (!fits) return false;
-        slot_cells = elem_bytes == 4 ? tile_slot_cells<float>(ge, tile_variant)
-                                     : tile_slot_cells<double>(ge, tile_variant);
-    } else {
-        if (bytes > kMaxTileBytes) return false;
-        if (d == 3 && W > 14) return false;
-    }
-    // the composite sort key must fit 32 bits
-    const uint64_t sr = planes() ? sub_range(bin_geom(*this)) : 1u;
-    const uint64_t kmax = (uint64_t)ntiles * sr;
-    if (kmax > (uint64_t(1) << 32)) return false;
-    int bits = 1;
-    while ((uint64_t(1) << bits) < kmax) ++bits;
-    sort_passes = (bits + 7) / 8;
-    usable = 1;
-    return true;
-}
-
-static size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
-
-// Offsets of the buffers in the binning's device block (carve == true: set
-// the pointers from base).  Sizes:
-//   keys, keys2, perm, perm2    M u32 each
-//   rs_hist                     256 x radix blocks u32
-//   scan_part                   2 x the blocks of the larger scan
-//   tile_count/_start, chunk_start  ntiles u32 each; n_chunks 2 (count, work counter)
-//   chunks                      max_chunks
-//   plane-tiled: desc, desc2    M descriptors each; slots, fs (own scratch)
-//   node-lane:   xs             M d doubles
-static size_t bin_layout(Binning &b, int64_t M, char *base)
-{
-    const int64_t nblk = (M + kRsItems - 1) / kRsItems;
-    const int64_t max_chunks = b.ntiles + (M + kChunk - 1) / kChunk;
-    const int64_t scan_n = std::max<int64_t>(b.ntiles, kRsDigits * nblk);
-    const size_t db = b.elem_bytes == 4 ? sizeof(NodeDesc<float>) : sizeof(NodeDesc<double>);
-    size_t off = 0;
-    auto take = [&](size_t bytes) {
-        char *p = base ? base + off : nullptr;
-        off += align256(bytes ? bytes : 16);
-        return p;
-    };
-    uint32_t *keys = (uint32_t *)take(4 * (size_t)M), *keys2 = (uint32_t *)take(4 * (size_t)M);
-    uint32_t *perm = (uint32_t *)take(4 * (size_t)M), *perm2 = (uint32_t *)take(4 * (size_t)M);
-    uint32_t *rs_hist = (uint32_t *)take(4 * (size_t)kRsDigits * nblk);
-    uint32_t *scan_part = (uint32_t *)take(4 * 2 * (size_t)((scan_n + kScanBlock - 1) / kScanBlock));
-    uint32_t *tile_count = (uint32_t *)take(4 * (size_t)b.ntiles);
-    uint32_t *tile_start = (uint32_t *)take(4 * (size_t)b.ntiles);
-    uint32_t *chunk_start = (uint32_t *)take(4 * (size_t)b.ntiles);
-    uint32_t *n_chunks = (uint32_t *)take(8);   // chunk count, then the spread's work counter
-    Chunk *chunks = (Chunk *)take(sizeof(Chunk) * (size_t)max_chunks);
-    void *desc = nullptr, *desc2 = nullptr, *slots = nullptr, *fs = nullptr;
-    double *xs = nullptr;
-    if (b.planes()) {
-        desc = take((size_t)M * db);
-        desc2 = take((size_t)M * db);
-        if (b.own_scratch) {
-            slots = take((size_t)max_chunks * b.slot_cells * 2 * b.elem_bytes);
-            fs = take((size_t)M * 2 * b.elem_bytes);
-        }
-    } else {
-        xs = (double *)take(sizeof(double) * (size_t)M * b.d);
-    }
-    if (base) {
-        b.keys = keys;
-        b.keys2 = keys2;
-        b.perm = perm;
-        b.perm2 = perm2;
-        b.rs_hist = rs_hist;
-        b.scan_part = scan_part;
-        b.tile_count = tile_count;
-        b.tile_start = tile_start;
-        b.chunk_start = chunk_start;
-        b.n_chunks = n_chunks;
-        b.chunks = chunks;
-        b.desc = desc;
-        b.desc2 = desc2;
-        b.slots = slots;
-        b.fs = fs;
-        b.xs = xs;
-        b.max_chunks = max_chunks;
-        b.M = M;
-    }
-    return off;
-}
-
-size_t Binning::bytes_for(int64_t M_) const { return bin_layout(const_cast<Binning &>(*this), M_, nullptr); }
-
-void Binning::carve(char *base, int64_t M_) { bin_layout(*this, M_, base); }
-
-bool Binning::bind(void *base, size_t bytes, int64_t M_)
-{
-    if (!usable || bytes < bytes_for(M_)) return false;
-    release();
-    block = base;
-    own_block = false;
-    carve(static_cast<char *>(base), M_);
-    return true;
-}
-
-// Scan of n counts cnt in place into their exclusive prefix (start == cnt
-// allowed) and, for tile counts, of their chunk counts into chunk_start.
-static void scan_counts(const uint32_t *cnt, uint32_t *start, uint32_t *chunk_start,
-                        uint32_t *n_chunks, uint32_t *part, int64_t n, hipStream_t s)
-{
-    const int64_t nparts = (n + kScanBlock - 1) / kScanBlock;
-    k_bin_scan_part<<<(unsigned)nparts, kScanBlock, 0, s>>>(cnt, part, n, nparts);
-    k_bin_scan_top<<<1, kScanBlock, 0, s>>>(part, nparts, n_chunks);
-    k_bin_scan_apply<<<(unsigned)nparts, kScanBlock, 0, s>>>(cnt, part, start, chunk_start, n, nparts);
-}
-
-// The binning passes: keys (and, for the plane-tiled kernels, descriptors by
-// node), the radix sort of the keys, the tile counts from the sorted keys,
-// tile scan and chunk list, and the sorted copies of the per-node data.
-template <typename T> void Binning::run_build(const Geom &ge, const BinGeom &bg, const double *x,
-                                              hipStream_t s)
-{
-    const unsigned gm = (unsigned)((M + 255) / 256);
-    NodeDesc<T> *dj = planes() ? static_cast<NodeDesc<T> *>(desc2) : nullptr;   // by node
-    const uint32_t sr = planes() ? sub_range(bg) : 1u;
-    k_fill_u32<<<(unsigned)((ntiles + 255) / 256), 256, 0, s>>>(tile_count, ntiles, 0u);
-    k_bin_keys<T><<<gm, 256, 0, s>>>(x, keys, dj, ge, bg, sr);
-    // radix passes: pass p reads (kin, vin) and writes (kout, vout); the
-    // destinations alternate so that the last pass writes perm
-    const uint32_t nblk = (uint32_t)((M + kRsItems - 1) / kRsItems);
-    uint32_t *kbuf[2] = {keys, keys2};
-    uint32_t *vbuf[2] = {perm, perm2};
-    uint32_t *skeys = nullptr;   // the sorted keys (written by the last pass)
-    for (int p = 0; p < sort_passes; ++p) {
-        const int dst = (sort_passes - 1 - p) & 1;   // the last pass writes buffer 0 (perm)
-        const uint32_t *kin = p == 0 ? keys : kbuf[dst ^ 1];
-        const uint32_t *vin = p == 0 ? nullptr : vbuf[dst ^ 1];
-        // the first pass reads keys (buffer 0); it must not also write keys;
-        // the last one writes its keys into whichever key buffer it does not read
-        uint32_t *kout = p + 1 < sort_passes ? (p == 0 ? keys2 : kbuf[dst]) : (kin == keys ? keys2 : keys);
-        if (p + 1 == sort_passes) skeys = kout;
-        uint32_t *vout = vbuf[dst];
-        k_rs_hist<<<nblk, kRsThreads, 0, s>>>(kin, M, 8 * p, rs_hist, nblk);
-        scan_counts(rs_hist, rs_hist, nullptr, nullptr, scan_part, (int64_t)kRsDigits * nblk, s);
-        k_rs_scatter<<<nblk, kRsThreads, 0, s>>>(kin, vin, M, 8 * p, rs_hist, nblk, kout, vout);
-        if (p == 0) {
-            // later passes ping-pong between keys2 and keys
-            kbuf[dst] = keys2;
-            kbuf[dst ^ 1] = keys;
-        }
-    }
-    // tile counts (tile_start holds each tile's first position until the scan
-    // overwrites it), then the scans and the chunk list
-    k_bin_tile_first<<<gm, 256, 0, s>>>(skeys, M, sr, tile_start);
-    k_bin_tile_count<<<gm, 256, 0, s>>>(skeys, M, sr, tile_start, tile_count);
-    scan_counts(tile_count, tile_start, chunk_start, n_chunks, scan_part, ntiles, s);
-    k_bin_chunks<<<(unsigned)((ntiles + 255) / 256), 256, 0, s>>>(tile_count, tile_start,
-                                                                  chunk_start, chunks, ntiles);
-    if (planes())
-        k_bin_gather_desc<T><<<gm, 256, 0, s>>>(perm, dj, static_cast<NodeDesc<T> *>(desc), M);
-    else
-        k_bin_gather_x<<<gm, 256, 0, s>>>(perm, x, xs, M, d);
-}
-
-void Binning::build(const Geom &ge, const double *x, hipStream_t s)
-{
-    if (!usable) return;
-    if (!block || M != ge.M) {
-        if (block && !own_block)
-            throw Error(CUNFFT_ERR_STATE, "bound binning memory is sized for another node count");
-        release();
-        const size_t bytes = bytes_for(ge.M);
-        void *p = nullptr;
-        CUNFFT_HIP(hipMalloc(&p, bytes));
-        block = p;
-        own_block = true;
-        carve(static_cast<char *>(p), ge.M);
-    }
-    const BinGeom bg = bin_geom(*this);
-    if (elem_bytes == 4) run_build<float>(ge, bg, x, s);
-    else run_build<double>(ge, bg, x, s);
-    CUNFFT_HIP(hipGetLastError());
-    built = 1;
-}
-
-void Binning::release()
-{
-    if (block && own_block) (void)hipFree(block);
-    block = nullptr;
-    own_block = false;
-    keys = keys2 = perm = perm2 = rs_hist = scan_part = nullptr;
-    tile_count = tile_start = chunk_start = n_chunks = nullptr;
-    chunks = nullptr;
-    xs = nullptr;
-    desc = desc2 = slots = fs = nullptr;
-    built = 0;
-    M = 0;
 }
 
 // ------------------------------------------------------ tile helpers ----

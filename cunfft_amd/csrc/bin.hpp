@@ -113,13 +113,14 @@ struct Binning {
     int64_t M = 0;
     int64_t max_chunks = 0;
     int64_t slot_cells = 0;     // padded-tile cells of one adjoint slot
-    int sort_passes = 0;        // radix passes (8-bit digits) over the composite key
+    int key_bits = 0;           // bits of the composite key
+    int sort_passes = 0;        // radix passes (digits of up to 8 bits) over it
     uint32_t *keys = nullptr;       // M: composite key of each node (node order), sort ping-pong
     uint32_t *keys2 = nullptr;      // M: sort ping-pong
     uint32_t *perm = nullptr;       // M: node at each sorted position
     uint32_t *perm2 = nullptr;      // M: sort ping-pong
-    uint32_t *rs_hist = nullptr;    // 256 x radix blocks: digit counts, then their offsets
-    uint32_t *scan_part = nullptr;  // block sums of the scans
+    uint32_t *rs_hist = nullptr;    // radix blocks x 256: digit counts, or their offsets
+    uint32_t *scan_part = nullptr;  // digit totals, then chunk sums of tile blocks
     uint32_t *tile_count = nullptr; // ntiles
     uint32_t *tile_start = nullptr; // ntiles
     uint32_t *chunk_start = nullptr;// ntiles

@@ -4,7 +4,24 @@
 
 namespace cunfft {
 
-constexpr int kChunk = 256;   // nodes per chunk (one workgroup's share of a tile)
+constexpr int kChunk = 256;   // nodes per chunk (one workgroup's share of a tile), at most
+constexpr int kChunkShift = 8, kChunkShiftMin = 5;   // chunks of 32 .. 256 nodes
+constexpr int kTileChunksAim = 16;   // chunks of a dense tile before they grow
+
+// log2 of the nodes per chunk of a tile with c nodes, from the binning's shift
+// base.  A tile with more than kTileChunksAim chunks takes larger ones, up to
+// kChunk: its fold adds the chunks one after the other.
+__host__ __device__ __forceinline__ int chunk_shift(uint32_t c, int base)
+{
+    int s = base;
+    while (s < kChunkShift && (c >> s) > (uint32_t)kTileChunksAim) ++s;
+    return s;
+}
+__host__ __device__ __forceinline__ uint32_t chunks_of(uint32_t c, int base)
+{
+    const int s = chunk_shift(c, base);
+    return (c + (1u << s) - 1u) >> s;
+}
 constexpr int kFoldSegBytes = 32;   // bytes of a core column one fold thread sums (FP32, d >= 2)
 
 // Grid tile per dimension: the nodes whose window starts in one tile are
@@ -33,7 +50,7 @@ inline void tile_shape(int d, int v, int64_t (&T)[3])
     for (int t = 0; t < 3; ++t) T[t] = shapes[d][v][t];
 }
 
-// Work item of the tiled kernels: up to kChunk sorted nodes of one tile.
+// Work item of the tiled kernels: up to 1 << chunk_shift sorted nodes of one tile.
 struct Chunk {
     uint32_t tile;
     uint32_t start;  // first sorted position
@@ -54,12 +71,22 @@ struct Chunk {
 // 7 (kXcdGroup - 1) chunks below b).
 constexpr uint32_t kXcds = 8;
 constexpr uint32_t kXcdGroup = 128;
-__host__ __device__ __forceinline__ int64_t xcd_chunk(uint32_t b, uint32_t n)
+__host__ __device__ __forceinline__ int64_t xcd_chunk(uint32_t b, uint32_t n, uint32_t group = kXcdGroup)
 {
     const uint32_t x = b % kXcds, local = b / kXcds;
-    const uint64_t g = (uint64_t)(local / kXcdGroup) * kXcds + x;
-    const uint64_t c = g * kXcdGroup + local % kXcdGroup;
+    const uint64_t g = (uint64_t)(local / group) * kXcds + x;
+    const uint64_t c = g * group + local % group;
     return c < n ? (int64_t)c : -1;
+}
+// Group length for n chunks: kXcdGroup from 8192 chunks on, below that the power
+// of two that gives every XCD at least 8 groups (with 128-chunk groups the 304
+// chunks of a 50021-node plan ran on 3 of the 8 XCDs).  A shorter group needs no
+// more workgroups than xcd_grid holds.
+__host__ __device__ __forceinline__ uint32_t xcd_group(uint32_t n)
+{
+    uint32_t g = kXcdGroup;
+    while (g > 1 && (uint64_t)g * kXcds * 8 > n) g >>= 1;
+    return g;
 }
 inline unsigned xcd_grid(int64_t max_chunks)
 {
@@ -111,6 +138,7 @@ struct Binning {
     int64_t nt[3] = {1, 1, 1};  // tiles per axis
     int64_t ntiles = 0;
     int64_t M = 0;
+    int chunk_base = kChunkShift;   // log2 of the nodes per chunk (chunk_shift)
     int64_t max_chunks = 0;
     int64_t slot_cells = 0;     // padded-tile cells of one adjoint slot
     int key_bits = 0;           // bits of the composite key
@@ -160,6 +188,7 @@ struct BinGeom {
     int64_t nt[3];
     int64_t ntiles;
     int sub_shift;   // column cells per lane unit, log2 (FP32 1, FP64 0)
+    int chunk_base;  // log2 of the nodes per chunk (chunk_shift)
 };
 
 // Order of a node within its tile (window start lo_t relative to the tile

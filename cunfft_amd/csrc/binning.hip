@@ -43,6 +43,7 @@ BinGeom bin_geom(const Binning &b)
     }
     g.ntiles = b.ntiles;
     g.sub_shift = b.elem_bytes == 4 ? 1 : 0;
+    g.chunk_base = b.chunk_base;
     return g;
 }
 
@@ -336,24 +337,23 @@ __device__ __forceinline__ uint32_t tile_nodes(const uint32_t *__restrict__ firs
 {
     return (t + 1 < ntiles ? first[t + 1] : M) - first[t];
 }
-__device__ __forceinline__ uint32_t chunks_of(uint32_t c) { return (c + kChunk - 1) / kChunk; }
 
 // part[b] = chunks of the tiles of workgroup b (more than kChunkDirect of them).
 __global__ __launch_bounds__(kTileBlock) void k_bin_chunk_part(const uint32_t *__restrict__ first,
-                                                               int64_t ntiles, uint32_t M,
+                                                               int64_t ntiles, uint32_t M, int base,
                                                                uint32_t *__restrict__ part)
 {
     __shared__ uint32_t ws[kTileBlock / 64];
     const int64_t t = (int64_t)blockIdx.x * kTileBlock + threadIdx.x;
     uint32_t all;
-    (void)block_exscan<kTileBlock>(t < ntiles ? chunks_of(tile_nodes(first, t, ntiles, M)) : 0u, ws, all);
+    (void)block_exscan<kTileBlock>(t < ntiles ? chunks_of(tile_nodes(first, t, ntiles, M), base) : 0u, ws, all);
     if (threadIdx.x == 0) part[blockIdx.x] = all;
 }
 
 // Tile counts, the first chunk of every tile, the chunk list and its length.
 // part NULL: the chunks of the tiles before the workgroup's are counted here.
 __global__ __launch_bounds__(kTileBlock) void k_bin_chunks(const uint32_t *__restrict__ first,
-                                                           int64_t ntiles, uint32_t M,
+                                                           int64_t ntiles, uint32_t M, int base,
                                                            const uint32_t *__restrict__ part,
                                                            uint32_t *__restrict__ count,
                                                            uint32_t *__restrict__ chunk_start,
@@ -368,24 +368,43 @@ __global__ __launch_bounds__(kTileBlock) void k_bin_chunks(const uint32_t *__res
         for (int64_t b = tid; b < (int64_t)blockIdx.x; b += kTileBlock) sum += part[b];
     } else {
 #pragma unroll 4
-        for (int64_t u = tid; u < t0; u += kTileBlock) sum += chunks_of(tile_nodes(first, u, ntiles, M));
+        for (int64_t u = tid; u < t0; u += kTileBlock) sum += chunks_of(tile_nodes(first, u, ntiles, M), base);
     }
     uint32_t before, all;
     (void)block_exscan<kTileBlock>(sum, ws, before);
     const uint32_t c = t < ntiles ? tile_nodes(first, t, ntiles, M) : 0u;
-    const uint32_t o0 = before + block_exscan<kTileBlock>(chunks_of(c), ws, all);
+    const uint32_t o0 = before + block_exscan<kTileBlock>(chunks_of(c, base), ws, all);
     if (t < ntiles) {
         count[t] = c;
         chunk_start[t] = o0;
         const uint32_t s0 = first[t];
         uint32_t o = o0;
-        for (uint32_t s = 0; s < c; s += kChunk, ++o)
-            chunks[o] = Chunk{(uint32_t)t, s0 + s, c - s < (uint32_t)kChunk ? c - s : (uint32_t)kChunk, 0u};
+        const uint32_t len = 1u << chunk_shift(c, base);
+        for (uint32_t s = 0; s < c; s += len, ++o)
+            chunks[o] = Chunk{(uint32_t)t, s0 + s, c - s < len ? c - s : len, 0u};
     }
-    if (t == ntiles - 1) n_chunks[0] = o0 + chunks_of(c);
+    if (t == ntiles - 1) n_chunks[0] = o0 + chunks_of(c, base);
 }
 
 // ------------------------------------------------------------------ host --
+// log2 of the nodes per chunk of a plan of M nodes.  A wavefront walks its chunk's
+// nodes one after the other, each a chain of LDS round trips, so with few nodes the
+// longest chunk sets the time and most CUs idle; a chunk costs the staging or the slot
+// of its padded tile, so with many nodes longer ones win.  Forward + adjoint in us at
+// 256 / 128 / 64 / 32 nodes per chunk:
+//   2D     4097 nodes  126 /  82 /  59 /  51       3D   30001 nodes  143 /  131 /  138 /  159
+//   2D    50021 nodes  332 / 218 / 172 / 164       3D   60001 nodes  510 /  423 /  437 /  471
+//   2D   100800 nodes  220 / 220 / 242 / 242       3D  400009 nodes 1090 / 1029 / 1062 / 1169
+//   2D   262144 nodes  182 / 188 / 211 / 222       3D  262145 nodes  646 /  643 /  705 /  797
+// Hence about 1024 chunks at most from splitting in 2D, and 128 nodes or more in 3D,
+// whose slots are larger.  A batch has its problems to fill the GPU: the longest chunks.
+static int plan_chunk_base(int d, int64_t M)
+{
+    int s = d == 3 ? 7 : kChunkShiftMin;
+    while (s < kChunkShift && (M >> s) > (d == 3 ? 4096 : 1024)) ++s;
+    return s;
+}
+
 bool Binning::plan(const Geom &ge, int elem_bytes_, int kernel_variant, int tile_variant_)
 {
     variant = kernel_variant;
@@ -409,6 +428,7 @@ bool Binning::plan(const Geom &ge, int elem_bytes_, int kernel_variant, int tile
         if (t < d) bytes *= T[t] + W - 1;
     }
     if (ntiles >= (int64_t(1) << 31)) return false;
+    chunk_base = planes() && own_scratch ? plan_chunk_base(d, ge.M) : kChunkShift;
     if (planes()) {
         // plane-tiled kernels: 32-bit grid offsets and the LDS tile must fit
         if (ncells > (int64_t(1) << 32)) return false;
@@ -449,7 +469,7 @@ static size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 static size_t bin_layout(Binning &b, int64_t M, char *base)
 {
     const int64_t nblk = rs_blocks(M);
-    const int64_t max_chunks = b.ntiles + (M + kChunk - 1) / kChunk;
+    const int64_t max_chunks = b.ntiles + ((M + (int64_t(1) << b.chunk_base) - 1) >> b.chunk_base);
     const int64_t nparts = (b.ntiles + kTileBlock - 1) / kTileBlock;
     const size_t db = b.elem_bytes == 4 ? sizeof(NodeDesc<float>) : sizeof(NodeDesc<double>);
     size_t off = 0;
@@ -588,8 +608,9 @@ template <typename T> void Binning::run_build(const Geom &ge, const BinGeom &bg,
         skeys, perm, M, sub_bits, (uint32_t)ntiles, dj, static_cast<NodeDesc<T> *>(desc), x, xs, d, tile_start);
     const int64_t nparts = (ntiles + kTileBlock - 1) / kTileBlock;
     if (nparts > kChunkDirect)
-        k_bin_chunk_part<<<(unsigned)nparts, kTileBlock, 0, s>>>(tile_start, ntiles, (uint32_t)M, scan_part);
-    k_bin_chunks<<<(unsigned)nparts, kTileBlock, 0, s>>>(tile_start, ntiles, (uint32_t)M,
+        k_bin_chunk_part<<<(unsigned)nparts, kTileBlock, 0, s>>>(tile_start, ntiles, (uint32_t)M, chunk_base,
+                                                                     scan_part);
+    k_bin_chunks<<<(unsigned)nparts, kTileBlock, 0, s>>>(tile_start, ntiles, (uint32_t)M, chunk_base,
                                                          nparts > kChunkDirect ? scan_part : nullptr,
                                                          tile_count, chunk_start, chunks, n_chunks);
 }

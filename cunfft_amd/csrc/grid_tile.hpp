@@ -574,6 +574,13 @@ __device__ __forceinline__ void stage_tile(const cplx_t<T> *__restrict__ g, uint
     }
 }
 
+// Nodes per batch of a wavefront: NB, or an equal share of a chunk too short to
+// give each of the NW wavefronts a full batch.
+template <int NB, int NW> __device__ __forceinline__ uint32_t node_batch(uint32_t count)
+{
+    return count >= (uint32_t)(NB * NW) ? (uint32_t)NB : (count + NW - 1) / NW;
+}
+
 // ------------------------------------------------------------ gather ----
 // NW wavefronts share the staged tile and take batches of the chunk's nodes
 // round-robin.  Each lane accumulates its unit over the node's planes and
@@ -598,14 +605,15 @@ __device__ __forceinline__ void tile_gather(const cplx_t<T> *__restrict__ g,
     __shared__ WinBatch<T, D, W, NB> wbs[NW];
     __shared__ C red[NW][NB][4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t nbat = (ch.count + NB - 1) / NB;
+    const uint32_t nbw = node_batch<NB, NW>(ch.count);
+    const uint32_t nbat = (ch.count + nbw - 1) / nbw;
 
     // this wavefront's first batch in flight while the tile is staged
     NodeDesc<T> nd{};
     uint32_t pm = 0;
     {
-        const uint32_t s = (uint32_t)wave * NB + lane;
-        if (lane < NB && s < ch.count) {
+        const uint32_t s = (uint32_t)wave * nbw + lane;
+        if ((uint32_t)lane < nbw && s < ch.count) {
             nd = desc[ch.start + s];
             pm = perm[ch.start + s];
         }
@@ -621,13 +629,13 @@ __device__ __forceinline__ void tile_gather(const cplx_t<T> *__restrict__ g,
     WinBatch<T, D, W, NB> &wb = wbs[wave];
 
     for (uint32_t bi = wave; bi < nbat; bi += NW) {
-        const uint32_t s0 = bi * NB;
-        const int nb = ch.count - s0 < (uint32_t)NB ? (int)(ch.count - s0) : NB;
+        const uint32_t s0 = bi * nbw;
+        const int nb = (int)(ch.count - s0 < nbw ? ch.count - s0 : nbw);
         const NodeRec rc = batch_prologue<T, D, W, NB, L>(wb, nb, lane, nd, wc);
         const uint32_t pm_out = pm;
         {
-            const uint32_t s = s0 + NW * NB + lane;
-            if (lane < NB && s < ch.count) {
+            const uint32_t s = s0 + NW * nbw + lane;
+            if ((uint32_t)lane < nbw && s < ch.count) {
                 nd = desc[ch.start + s];
                 pm = perm[ch.start + s];
             }
@@ -718,7 +726,8 @@ __global__ __launch_bounds__(NW * 64) void k_tile_gather(
     const uint32_t *__restrict__ n_chunks, cplx_t<T> *__restrict__ f, Geom ge, BinGeom bg,
     WinConst<T> wc)
 {
-    const int64_t c = xcd_chunk(blockIdx.x, n_chunks[0]);
+    const uint32_t n = n_chunks[0];
+    const int64_t c = xcd_chunk(blockIdx.x, n, xcd_group(n));
     if (c < 0) return;
     tile_gather<T, D, W, NW, V>(g, desc, perm, chunks[c], f, ge, bg, wc);
 }
@@ -819,13 +828,14 @@ __device__ __forceinline__ void tile_grad(const cplx_t<T> *__restrict__ g,
     __shared__ DwBatch<T, D, W, NB> dbs[NW];
     __shared__ C red[NW][NB][4][D];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t nbat = (ch.count + NB - 1) / NB;
+    const uint32_t nbw = node_batch<NB, NW>(ch.count);
+    const uint32_t nbat = (ch.count + nbw - 1) / nbw;
 
     NodeDesc<T> nd{};
     uint32_t pm = 0;
     {
-        const uint32_t s = (uint32_t)wave * NB + lane;
-        if (lane < NB && s < ch.count) {
+        const uint32_t s = (uint32_t)wave * nbw + lane;
+        if ((uint32_t)lane < nbw && s < ch.count) {
             nd = desc[ch.start + s];
             pm = perm[ch.start + s];
         }
@@ -841,14 +851,14 @@ __device__ __forceinline__ void tile_grad(const cplx_t<T> *__restrict__ g,
     DwBatch<T, D, W, NB> &db = dbs[wave];
 
     for (uint32_t bi = wave; bi < nbat; bi += NW) {
-        const uint32_t s0 = bi * NB;
-        const int nb = ch.count - s0 < (uint32_t)NB ? (int)(ch.count - s0) : NB;
+        const uint32_t s0 = bi * nbw;
+        const int nb = (int)(ch.count - s0 < nbw ? ch.count - s0 : nbw);
         const NodeRec rc = batch_prologue<T, D, W, NB, L>(wb, nb, lane, nd, wc);
         dw_prologue<T, D, W, NB>(db, wb, nb, lane, wc);
         const uint32_t pm_out = pm;
         {
-            const uint32_t s = s0 + NW * NB + lane;
-            if (lane < NB && s < ch.count) {
+            const uint32_t s = s0 + NW * nbw + lane;
+            if ((uint32_t)lane < nbw && s < ch.count) {
                 nd = desc[ch.start + s];
                 pm = perm[ch.start + s];
             }
@@ -964,7 +974,8 @@ __global__ __launch_bounds__(NW * 64) void k_tile_grad(
     const uint32_t *__restrict__ n_chunks, const cplx_t<T> *__restrict__ v, T *__restrict__ gx, Geom ge,
     BinGeom bg, WinConst<T> wc)
 {
-    const int64_t c = xcd_chunk(blockIdx.x, n_chunks[0]);
+    const uint32_t n = n_chunks[0];
+    const int64_t c = xcd_chunk(blockIdx.x, n, xcd_group(n));
     if (c < 0) return;
     tile_grad<T, D, W, NW, V>(g, desc, perm, chunks[c], v, gx, ge, bg, wc);
 }
@@ -1603,7 +1614,7 @@ __device__ __forceinline__ void tile_fold(const cplx_t<T> *__restrict__ slots,
             }
             const uint32_t cnt = tile_count[src];
             c0[qq] = chunk_start[src];
-            nch[qq] = (cnt + kChunk - 1) / kChunk;
+            nch[qq] = chunks_of(cnt, bg.chunk_base);
             const int boff = L::block_off(q0, q1, qL);
 #pragma unroll
             for (int k = 0; k < CPT; ++k) {
@@ -1762,7 +1773,7 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
                 const uint32_t src = ((tk[0] + 4 * n0 - q0) % n0 * n1 + (tk[1] + 4 * n1 - q1) % n1) * n2 +
                                      (tk[2] + 4 * n2 - qL) % n2;
                 c0[q0][q1][qL] = chunk_start[src];
-                nch[q0][q1][qL] = (tile_count[src] + kChunk - 1) / kChunk;
+                nch[q0][q1][qL] = chunks_of(tile_count[src], bg.chunk_base);
             }
     T sx[SEGC], sy[SEGC], cx[SEGC], cy[SEGC];
 #pragma unroll
@@ -1812,22 +1823,30 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
                         fold_add<COMP>(sy[i], cy[i], v[qL][i].y);
                     }
             }
-            // further chunks of dense candidate tiles
+            // further chunks of dense candidate tiles, four loads in flight
 #pragma unroll
             for (int qL = 0; qL < QL; ++qL) {
                 const int EL = L::ext(TL, L::PL, qL);
                 const int o = L::block_off(q0, q1, qL) + rc * EL;
-                for (uint32_t c = 1; c < nch[q0][q1][qL]; ++c) {
-                    const C *sp = slots + (int64_t)(c0[q0][q1][qL] + c) * L::SC;
-                    C w[SEGC];
-                    if (EL == TL) load_full(sp, o + seg * SEGC, w);
-                    else load_last(sp, o, w);
+                const uint32_t nc = nch[q0][q1][qL];
+                for (uint32_t c = 1; c < nc; c += 4) {
+                    C w[4][SEGC];
 #pragma unroll
-                    for (int i = 0; i < SEGC; ++i)
-                        if ((EL == TL || (i < NLAST && seg * SEGC + i < EL)) && in01) {
-                            fold_add<COMP>(sx[i], cx[i], w[i].x);
-                            fold_add<COMP>(sy[i], cy[i], w[i].y);
-                        }
+                    for (int u = 0; u < 4; ++u) {
+                        // past the last chunk: the last one again, not added
+                        const uint32_t cu = c + u < nc ? c + u : nc - 1;
+                        const C *sp = slots + (int64_t)(c0[q0][q1][qL] + cu) * L::SC;
+                        if (EL == TL) load_full(sp, o + seg * SEGC, w[u]);
+                        else load_last(sp, o, w[u]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+#pragma unroll
+                        for (int i = 0; i < SEGC; ++i)
+                            if ((EL == TL || (i < NLAST && seg * SEGC + i < EL)) && in01 && c + u < nc) {
+                                fold_add<COMP>(sx[i], cx[i], w[u][i].x);
+                                fold_add<COMP>(sy[i], cy[i], w[u][i].y);
+                            }
                 }
             }
         }

@@ -1036,7 +1036,12 @@ int api_adjoint_noalloc_dev(typename Traits<T>::plan *p, const void *f, void *fh
         Binning b;   // describes the scratch; owns nothing
         if (!(p->flags & CUNFFT_ATOMIC_SCATTER) &&
             plan_bins(b, im->geom, (int)sizeof(T), im->config[1], im->compensated)) {
-            const size_t need = b.bytes_for(p->M_total);
+            size_t need = b.bytes_for(p->M_total);
+            if (need > kNoAllocScratchBytes) {
+                // the fewest slots: the longest chunks
+                b.chunk_base = kChunkShift;
+                need = b.bytes_for(p->M_total);
+            }
             if (need > kNoAllocScratchBytes) {
                 char msg[200];
                 snprintf(msg, sizeof msg,

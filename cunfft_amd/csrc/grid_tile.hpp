@@ -191,9 +191,10 @@ template <typename T, int D, int W, int PS, int V> struct TileLayout {
 
 // The Kaiser-Bessel and sinc weights out of line: the Gaussian path keeps its
 // registers (the window is a run-time choice of the plan).
-template <typename T> __device__ __noinline__ T alt_phi_call(int win, T s, int m, T shape)
+template <typename T, bool GRAD> __device__ __noinline__ T alt_phi_call(int win, T s, int m, T shape)
 {
-    return win == WIN_SINC ? sinc_phi<T>(s, m, shape) : kb_phi<T>(s, (T)m, shape);
+    if (win == WIN_SINC) return sinc_phi<T>(s, m, shape);
+    return GRAD ? kb_phi_grad(s, (T)m, shape) : kb_phi<T>(s, (T)m, shape);
 }
 
 template <typename T> __device__ __forceinline__ T wexp(T v);
@@ -314,7 +315,7 @@ struct NodeRec {
 // its record and axis offsets, then every lane evaluates window weights.
 // Within one wavefront LDS accesses execute in order, so the compiler
 // barriers suffice between the phases.
-template <typename T, int D, int W, int NB, typename L, int NWP = 0>
+template <typename T, int D, int W, int NB, typename L, int NWP = 0, bool GRAD = false>
 __device__ __forceinline__ NodeRec batch_prologue(WinBatch<T, D, W, NB, NWP> &wb, int nb, int lane,
                                                   const NodeDesc<T> &nd, const WinConst<T> &wc)
 {
@@ -364,7 +365,7 @@ __device__ __forceinline__ NodeRec batch_prologue(WinBatch<T, D, W, NB, NWP> &wb
         for (int ps = 0; ps < NPASS; ++ps) {
             if (lane + 64 * ps >= nb * W) break;
             const T w = wc.win != WIN_GAUSSIAN
-                            ? alt_phi_call<T>(wc.win, sv[ps], wc.m, wc.shp[t])
+                            ? alt_phi_call<T, GRAD && sizeof(T) == 4>(wc.win, sv[ps], wc.m, wc.shp[t])
                             : wc.nrm[t] * wexp<T>(-wc.kb[t] * sv[ps] * sv[ps]);
             if (t == 0) {
                 if constexpr (NWP > 0)
@@ -450,7 +451,7 @@ __device__ __forceinline__ NodeRec batch_prologue_wg(WinBatch<T, D, W, NB, NWP> 
             const T kbt = t == 0 ? wc.kb[0] : (t == 1 ? wc.kb[1] : wc.kb[2]);
             const T nrt = t == 0 ? wc.nrm[0] : (t == 1 ? wc.nrm[1] : wc.nrm[2]);
             const T shpt = t == 0 ? wc.shp[0] : (t == 1 ? wc.shp[1] : wc.shp[2]);
-            const T w = wc.win != WIN_GAUSSIAN ? alt_phi_call<T>(wc.win, sv, wc.m, shpt)
+            const T w = wc.win != WIN_GAUSSIAN ? alt_phi_call<T, false>(wc.win, sv, wc.m, shpt)
                                                : nrt * wexp<T>(-kbt * sv * sv);
             if (t == 0) {
                 if constexpr (NWP > 0) wb.w0[n][(l % NWP) * WB::OWNP + l / NWP] = w;
@@ -853,7 +854,7 @@ __device__ __forceinline__ void tile_grad(const cplx_t<T> *__restrict__ g,
     for (uint32_t bi = wave; bi < nbat; bi += NW) {
         const uint32_t s0 = bi * nbw;
         const int nb = (int)(ch.count - s0 < nbw ? ch.count - s0 : nbw);
-        const NodeRec rc = batch_prologue<T, D, W, NB, L>(wb, nb, lane, nd, wc);
+        const NodeRec rc = batch_prologue<T, D, W, NB, L, 0, true>(wb, nb, lane, nd, wc);
         dw_prologue<T, D, W, NB>(db, wb, nb, lane, wc);
         const uint32_t pm_out = pm;
         {

@@ -6,16 +6,17 @@ namespace cunfft {
 
 constexpr int kChunk = 256;   // nodes per chunk (one workgroup's share of a tile), at most
 constexpr int kChunkShift = 8, kChunkShiftMin = 5;   // chunks of 32 .. 256 nodes
-constexpr int kTileChunksAim = 16;   // chunks of a dense tile before they grow
+constexpr int kTileChunksLog = 4;    // a dense tile's chunks grow at 16 of them
 
 // log2 of the nodes per chunk of a tile with c nodes, from the binning's shift
-// base.  A tile with more than kTileChunksAim chunks takes larger ones, up to
-// kChunk: its fold adds the chunks one after the other.
+// base.  A tile that would have 1 << kTileChunksLog chunks takes larger ones, up to
+// kChunk: its fold adds the chunks one after the other.  (No loop: the fold works it
+// out for each of up to 27 candidate tiles.)
 __host__ __device__ __forceinline__ int chunk_shift(uint32_t c, int base)
 {
-    int s = base;
-    while (s < kChunkShift && (c >> s) > (uint32_t)kTileChunksAim) ++s;
-    return s;
+    const int need = 32 - kTileChunksLog - __builtin_clz(c | 1u);   // c >> need < 1 << kTileChunksLog
+    const int s = need > base ? need : base;
+    return s < kChunkShift ? s : kChunkShift;
 }
 __host__ __device__ __forceinline__ uint32_t chunks_of(uint32_t c, int base)
 {
@@ -139,6 +140,7 @@ struct Binning {
     int64_t ntiles = 0;
     int64_t M = 0;
     int chunk_base = kChunkShift;   // log2 of the nodes per chunk (chunk_shift)
+    int seg_shift = 0;          // log2 of the chunks per chain of the matrix-core spread
     int64_t max_chunks = 0;
     int64_t slot_cells = 0;     // padded-tile cells of one adjoint slot
     int key_bits = 0;           // bits of the composite key
@@ -189,6 +191,7 @@ struct BinGeom {
     int64_t ntiles;
     int sub_shift;   // column cells per lane unit, log2 (FP32 1, FP64 0)
     int chunk_base;  // log2 of the nodes per chunk (chunk_shift)
+    int seg_shift;   // log2 of the chunks per chain (ChainSlot)
 };
 
 // Order of a node within its tile (window start lo_t relative to the tile

@@ -44,6 +44,7 @@ BinGeom bin_geom(const Binning &b)
     g.ntiles = b.ntiles;
     g.sub_shift = b.elem_bytes == 4 ? 1 : 0;
     g.chunk_base = b.chunk_base;
+    g.seg_shift = b.seg_shift;
     return g;
 }
 
@@ -397,12 +398,34 @@ __global__ __launch_bounds__(kTileBlock) void k_bin_chunks(const uint32_t *__res
 //   2D   100800 nodes  220 / 220 / 242 / 242       3D  400009 nodes 1090 / 1029 / 1062 / 1169
 //   2D   262144 nodes  182 / 188 / 211 / 222       3D  262145 nodes  646 /  643 /  705 /  797
 // Hence about 1024 chunks at most from splitting in 2D, and 128 nodes or more in 3D,
-// whose slots are larger.  A batch has its problems to fill the GPU: the longest chunks.
-static int plan_chunk_base(int d, int64_t M)
+// whose slots are larger: there only where no evenly filled tile is split (at 123 nodes
+// per tile, where a third would be, 342 us instead of 293).  A batch has its problems
+// to fill the GPU: the longest chunks.
+static int plan_chunk_base(int d, int64_t M, int64_t ntiles)
 {
-    int s = d == 3 ? 7 : kChunkShiftMin;
-    while (s < kChunkShift && (M >> s) > (d == 3 ? 4096 : 1024)) ++s;
+    if (d == 3) return M <= 80 * ntiles && (M >> 7) <= 4096 ? 7 : kChunkShift;
+    int s = kChunkShiftMin;
+    while (s < kChunkShift && (M >> s) > 1024) ++s;
     return s;
+}
+
+// log2 of the chunks per chain of the 3D matrix-core spread.  A chain of k tiles writes
+// (9 k + 8) / (17 k) of the slots that single chunks write (W = 10) and is one
+// workgroup's work in one piece.  Forward + adjoint (the adjoint at m = 6) in us for
+// chains of 1 / 2 / 4 / 8 chunks:
+//   FP32 256^3 grid, 2^21 nodes     1645 / 1549 / 1570 / 1675
+//   FP32  64^3 grid,  30001 nodes    133 /  125 /  141 /  173
+//   FP64 256^3 grid, 2^21 nodes     4390 / 4149 / 4051 / 4119
+//   FP64 128^3 grid, 262145 nodes    661 /  622 /  643 /  671
+//   FP64 128^3 grid, 2^18, m = 6     559 /  533 /  527 /  655
+//   FP64  64^3 grid,  60001, m = 6   317 /  319 /  397 /  494
+//   FP32 / FP64 128 x 64 x 64 grid, 122881 nodes, m = 4   93 / 117, 100 / 134, 115 / 157
+//   FP64 256 x 64 x 64 grid, 245761 nodes, m = 3         133 /  138 /  153
+// So two from 4096 tiles on (8 chains and more per resident FP64 workgroup), four for
+// FP64 from 16384; below, the chains leave workgroups idle at the end.
+static int plan_seg_shift(int elem_bytes, int64_t ntiles)
+{
+    return ntiles < 4096 ? 0 : elem_bytes == 8 && ntiles >= 16384 ? 2 : 1;
 }
 
 bool Binning::plan(const Geom &ge, int elem_bytes_, int kernel_variant, int tile_variant_)
@@ -428,7 +451,8 @@ bool Binning::plan(const Geom &ge, int elem_bytes_, int kernel_variant, int tile
         if (t < d) bytes *= T[t] + W - 1;
     }
     if (ntiles >= (int64_t(1) << 31)) return false;
-    chunk_base = planes() && own_scratch ? plan_chunk_base(d, ge.M) : kChunkShift;
+    chunk_base = planes() && own_scratch ? plan_chunk_base(d, ge.M, ntiles) : kChunkShift;
+    seg_shift = planes() && own_scratch ? plan_seg_shift(elem_bytes, ntiles) : 0;
     if (planes()) {
         // plane-tiled kernels: 32-bit grid offsets and the LDS tile must fit
         if (ncells > (int64_t(1) << 32)) return false;

@@ -22,9 +22,12 @@
 // * Planes.  The padded tile has P = 8 + W - 1 planes (17 at W = 10) but one
 //   instruction covers 16.  A node's window spans W planes from its start
 //   lo_0 in [0, 8), so the nodes are split into two sets: lo_0 <= 16 - W
-//   (window inside planes [0, 16)) and the rest (inside [P - 16, P)).  Each
+//   (window inside planes [0, 16)) and lo_0 >= P - 16 (inside [P - 16, P)).  Each
 //   set has its own accumulators whose rows are its 16 planes, and each node
-//   goes through the matrix cores once.  The sets are summed at the end.
+//   goes through the matrix cores once.  The sets are summed at the end.  At
+//   W = 14 the starts 3 and 4 fit neither set: such a node is in both, with its
+//   planes below 16 in the first and the others in the second (a quarter of uniform
+//   nodes, 1.25 products per node).
 // * Columns.  Each wavefront owns a band of rows b.  Per row it holds two
 //   blocks of 16 columns (columns c in [0, 8) and [8, 16), re/im), and the
 //   columns c >= 16 of all rows (P - 16 of them) are packed into extra
@@ -41,6 +44,14 @@
 //   destination-blocked order), which the workgroup then copies out with
 //   16-byte stores: whole cache lines, where storing the accumulators
 //   directly (4-byte lanes, 64-byte runs) took more than the matrix work.
+// * Chains.  Writing a whole padded tile per chunk (17^3 cells for 8^3) and reading
+//   it back in the fold is most of the adjoint's memory traffic.  A workgroup takes
+//   segments of 2^seg_shift consecutive chunks and keeps its accumulators from one
+//   to the next: for the same tile as they are; for the next tile along the last
+//   axis the columns [8, 16) become the new tile's [0, 8) (a register move: a lane
+//   holds the same column of both halves) and only the finished columns, 9 of 17,
+//   are written.  Segment ends and gaps in the tile row write everything.  The fold
+//   knows from the counts which slot parts hold a sum (ChainSlot).
 //
 // The sums per cell run over the nodes of the chunk in a fixed order (sorted
 // order within a set, in the instruction's fixed reduction order), so the
@@ -79,7 +90,8 @@ template <typename R, int W> struct MfmaSpread {
     static constexpr int P = T + W - 1;                 // padded extent per axis
     static constexpr int OFF1 = P > 16 ? P - 16 : 0;    // first plane of the second set
     static constexpr bool SETS2 = OFF1 > 0;
-    static constexpr int LO_MAX0 = 16 - W;              // set 0: window starts lo_0 <= LO_MAX0
+    static constexpr int LO_MAX0 = 16 - W;              // set 0 alone: window starts lo_0 <= LO_MAX0
+    static constexpr bool DUP = LO_MAX0 + 1 < OFF1;     // starts in (LO_MAX0, OFF1): both sets
     // wavefronts per workgroup: FP64 accumulators take twice the registers, so
     // twice the wavefronts share a tile's rows
     static constexpr int NW = sizeof(R) == 8 ? 8 : 4;
@@ -88,12 +100,14 @@ template <typename R, int W> struct MfmaSpread {
     static constexpr int NLOB = (P * NLO * 2 + 15) / 16;   // their 16-column blocks
     static constexpr int LB = (NLOB + NW - 1) / NW;     // of those, per wavefront (at most)
     static constexpr int NB = 32;                       // nodes per batch
-    static constexpr int NPOS = NB + 8;                 // batch rows: each set padded to 4 nodes
-    static constexpr int RS = 20;                       // row / column weight table stride
+    // batch rows: each set padded to 4 nodes, and one step past the last
+    static constexpr int NPOS = (DUP ? 2 * NB : NB) + 8;
+    static constexpr int RS = P <= 20 ? 20 : 24;        // row / column weight table stride
     // one table row per batch position: plane weights [0, 16), row weights times the
     // coefficient (re, im) from O_B1, column weights from O_B2; 80 floats, so the
-    // four rows one step reads start 16 banks apart
-    static constexpr int O_B1 = 16, O_B2 = O_B1 + 2 * RS, ROW = 80;
+    // four rows one step reads start 16 banks apart (88 for the wider rows of W = 14:
+    // 24 apart)
+    static constexpr int O_B1 = 16, O_B2 = O_B1 + 2 * RS, ROW = RS == 20 ? 80 : 88;
     static_assert(O_B2 + RS <= ROW, "a table row holds its four parts");
     // wavefront w: rows [row0(w), row0(w) + rows(w)) and extra(w) extra blocks
     static constexpr int row0(int w) { return w * P / NW; }
@@ -118,59 +132,48 @@ template <typename R, int W> struct MfmaSpread {
         for (int w = 0; w < NW; ++w) any = any || (rows(w) == nr && extra(w) == nl);
         return any;
     }
-    static_assert(W >= 2 && 2 * W + T <= 32, "every window start fits one of the two plane sets");
+    static_assert(W >= 2 && W <= 16 && OFF1 <= 7, "every window plane is in one of the two plane sets");
     static_assert(P <= RS, "a padded row fits the weight table stride");
 };
 
-template <typename R, int W> constexpr bool kMfmaSpread = W >= 4 && W <= 12;
+template <typename R, int W> constexpr bool kMfmaSpread = W >= 4 && W <= 14;
 // threads and resident workgroups per CU the kernel is built for
 template <typename R> constexpr int kMfmaThreads = sizeof(R) == 8 ? 512 : 256;
-template <typename R> constexpr int kMfmaPerCu = sizeof(R) == 8 ? 1 : 3;
+template <typename R, int W>
+constexpr int kMfmaPerCu = sizeof(R) == 8 ? 1 : (W <= 10 ? 3 : 2);
 
-// Element offset (units of R) of part ri of cell (a, b, c) in a slot of the
-// 8^3 padded tile (the destination-blocked order of TileLayout::block_off).
-template <typename L> __device__ __forceinline__ int mfma_slot_off(int a, int b, int c, int ri)
+// Part ri of cell (a, b, c) in the LDS image of the part of a chain slot (ChainSlot)
+// that starts at cell `from`, units of R.
+template <typename L> __device__ __forceinline__ int mfma_slot_off(int a, int b, int c, int ri, int from)
 {
     const int q1 = b >> 3, qL = c >> 3;
     const int E1 = L::ext(L::T1, L::P1, q1), EL = L::ext(L::TL, L::PL, qL);
-    return 2 * (L::block_off(a >> 3, q1, qL) + ((a & 7) * E1 + (b & 7)) * EL + (c & 7)) + ri;
+    return 2 * (ChainSlot<L>::off(a >> 3, q1, qL) - from + ((a & 7) * E1 + (b & 7)) * EL + (c & 7)) + ri;
 }
 
-// Float offsets in a slot of the 8^3 padded tile (the destination-blocked
-// order of TileLayout::block_off) of part ri of the cells (a, b, c) a lane
-// group g stores: planes a = 4g + i (i < 4, a < 16) at base + i * step, and
-// the planes a = 16 + i past them at base16 + i * step.
-struct MfmaSlotCol {
-    int base, base16, step;
-};
-template <typename L> __device__ __forceinline__ MfmaSlotCol mfma_slot_col(int g, int b, int c, int ri)
-{
-    const int q1 = b >> 3, qL = c >> 3;
-    const int E1 = L::ext(L::T1, L::P1, q1), EL = L::ext(L::TL, L::PL, qL);
-    const int in = (b & 7) * EL + (c & 7);   // row and column within the block
-    MfmaSlotCol o;
-    o.base = 2 * (L::block_off(g >> 1, q1, qL) + 4 * (g & 1) * E1 * EL + in) + ri;
-    o.base16 = 2 * (L::block_off(2, q1, qL) + in) + ri;
-    o.step = 2 * E1 * EL;
-    return o;
-}
-
-// Persistent: a grid of resident workgroups takes chunks from the work
-// counter n_chunks[1] (zero at launch) until it runs past the chunk count
-// n_chunks[0].  A workgroup holds the tickets of its current and its next
-// chunk and takes a third while the current one runs, so the next chunk's
+// Persistent: a grid of resident workgroups takes segments of 2^seg_shift chunks
+// from the work counter n_chunks[1] (zero at launch) until it runs past the chunk
+// count n_chunks[0].  A workgroup holds the tickets of its current and its next
+// segment and takes a third while the current one runs, so the next chunk's
 // record is in registers when its first batch is loaded; it exits at its
 // first ticket past the last chunk (its tickets rise, so every chunk below
 // the count is run).  The next batch's nodes (or the next chunk's first
 // batch) load while the current one runs through the matrix cores, and the
 // operands of the next 4-node step load while the current step's
 // instructions issue.
+//
+// Measured (256^3 grid, 2^21 nodes half clustered, W = 10; spread and fold): FP32
+// 631 + 366 -> 614 + 281 us, FP64 1619 + 697 -> 1496 + 539 us by the chains, the order
+// of the segments and image offsets computed where they are used.  W = 14 (128^3 grid,
+// 2^18 uniform nodes, FP64), which ran on the VALU with one workgroup per CU:
+// 912 + 122 -> 395 + 106 us.
+//
 // WIN: the window (inline, no calls: the accumulators stay in registers
 // through the weight evaluation).
 template <typename R, int W, int WIN>
-__global__ __launch_bounds__(kMfmaThreads<R>, kMfmaPerCu<R>) void k_tile_spread_mfma(
+__global__ __launch_bounds__(kMfmaThreads<R>, (kMfmaPerCu<R, W> * kMfmaThreads<R> / 256)) void k_tile_spread_mfma(
     const NodeDesc<R> *__restrict__ desc, const cplx_t<R> *__restrict__ fs, const Chunk *__restrict__ chunks,
-    uint32_t *__restrict__ n_chunks, cplx_t<R> *__restrict__ slots, WinConst<R> wc)
+    uint32_t *__restrict__ n_chunks, cplx_t<R> *__restrict__ slots, WinConst<R> wc, int seg_shift, uint32_t ntl)
 {
     using S = MfmaSpread<R, W>;
     using M = Mfma<R>;
@@ -183,7 +186,12 @@ __global__ __launch_bounds__(kMfmaThreads<R>, kMfmaPerCu<R>) void k_tile_spread_
     static_assert(L::T0 == S::T && L::T1 == S::T && L::TL == S::T && L::P0 == S::P, "8^3 tiles");
     constexpr int LBN = S::LB > 0 ? S::LB : 1;
     __shared__ __align__(16) R tw[S::NPOS][S::ROW];
-    __shared__ __align__(16) R stg[2 * L::SC];   // the slot image
+    // the slot image; where it does not fit (W = 14), the columns [8, 16) of a chain's
+    // end and the finished columns go one after the other through the same memory
+    using CS = ChainSlot<L>;
+    constexpr bool ONE = S::P <= 20;
+    constexpr int REST = L::SC - CS::HALF1, FROM0 = ONE ? 0 : CS::HALF1;
+    __shared__ __align__(16) R stg[2 * (ONE ? L::SC : CS::HALF1 > REST ? CS::HALF1 : REST)];
     __shared__ uint32_t s_tk[2];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -205,13 +213,29 @@ __global__ __launch_bounds__(kMfmaThreads<R>, kMfmaPerCu<R>) void k_tile_spread_
         lb_c[j] = lb_ok[j] ? 16 + e % (S::NLO > 0 ? S::NLO : 1) : 0;
     }
     uint32_t *counter = n_chunks + 1;
-    const uint32_t n = n_chunks[0];
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)n_chunks[0]);
     if (tid == 0) {
         s_tk[0] = atomicAdd(counter, 1u);
         s_tk[1] = atomicAdd(counter, 1u);
     }
     __syncthreads();
-    uint32_t c = s_tk[0], cn = s_tk[1];
+    const uint32_t segm = (1u << seg_shift) - 1u;   // chunk index within its segment
+    // First chunk of the segment of a ticket (n: none).  Segments are taken from the
+    // middle of the tile order on: windows that start near x = 0 are in the order's
+    // first and last tiles, and node sets dense around the origin would leave their
+    // longest segments for the end, when most workgroups have nothing left.
+    const uint32_t nseg = (n + segm) >> seg_shift;
+    auto first_chunk = [&](uint32_t tk) {
+        if (tk >= nseg) return n;
+        const uint32_t g = tk + (nseg >> 1);
+        return (g < nseg ? g : g - nseg) << seg_shift;
+    };
+    // (in scalar registers, like the chunk records: what the workgroup does next hangs
+    // on them, and a branch on them is then a scalar one)
+    auto ticket_at = [&](int k) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tk[k]); };
+    uint32_t c = first_chunk(ticket_at(0)), nxt = first_chunk(ticket_at(1));   // nxt: the next segment's
+    auto after = [&](uint32_t k) { return ((k + 1) & segm) != 0 && k + 1 < n ? k + 1 : nxt; };
+    uint32_t cn = after(c);
     // lanes n and n + 32: node n of the next batch to run (the two halves of a
     // wavefront share the weight evaluation of a node)
     static_assert(S::NB == 32, "a batch fills half a wavefront");
@@ -244,8 +268,10 @@ __global__ __launch_bounds__(kMfmaThreads<R>, kMfmaPerCu<R>) void k_tile_spread_
     // FP64 Gaussian: a quad's weights from two exps,
     // exp(-b (s0 - u)^2) = exp(-b s0^2) exp(2 b s0)^u exp(-b u^2), with the last
     // factor per axis (s0 is at most m + 4 in magnitude where a weight is used,
-    // so neither factor leaves the FP64 range)
-    constexpr bool GQUAD = WIN == WIN_GAUSSIAN && sizeof(R) == 8;
+    // so neither factor leaves the FP64 range).  W = 14 takes an exp per weight, as the
+    // VALU spread it replaces: the quads cost it a tenth of its accuracy (1.2e-15
+    // against 1.1e-15 of the adjoint) and save 20 us of 532.
+    constexpr bool GQUAD = WIN == WIN_GAUSSIAN && sizeof(R) == 8 && W <= 12;
     R gq1 = (R)1, gq2 = (R)1, gq3 = (R)1;
     if constexpr (GQUAD) {
         const int ax = wave / PW < 3 ? wave / PW : 2;
@@ -366,16 +392,18 @@ __global__ __launch_bounds__(kMfmaThreads<R>, kMfmaPerCu<R>) void k_tile_spread_
             if constexpr (S::SETS2) run(ks0, ks1, acc1, accL1);
         };
         uint32_t ticket = 0;
+#pragma unroll
+        for (int r = 0; r < S::RW; ++r) acc0[r][0] = acc0[r][1] = acc1[r][0] = acc1[r][1] = z4;
+#pragma unroll
+        for (int j = 0; j < LBN; ++j) accL0[j] = accL1[j] = z4;
+        bool busy = false;   // the weight tables may still be read (no barrier since the last step)
         while (c < n) {
-#pragma unroll
-            for (int r = 0; r < S::RW; ++r) acc0[r][0] = acc0[r][1] = acc1[r][0] = acc1[r][1] = z4;
-#pragma unroll
-            for (int j = 0; j < LBN; ++j) accL0[j] = accL1[j] = z4;
-            if (tid == 0) ticket = atomicAdd(counter, 1u);
+            if (tid == 0 && (c & segm) == 0) ticket = atomicAdd(counter, 1u);
             for (uint32_t s0 = 0; s0 < ch.count; s0 += S::NB) {
                 const int nb = __builtin_amdgcn_readfirstlane(
                     ch.count - s0 < (uint32_t)S::NB ? (int)(ch.count - s0) : S::NB);
-                if (s0 > 0) __syncthreads();   // every wavefront is done with the previous batch's tables
+                if (busy) __syncthreads();   // every wavefront is done with the previous batch's tables
+                busy = true;
                 const bool valid = nl < nb;
                 // the batch's node, loaded one batch ahead: opaque from here on, so
                 // no use of it is moved up to its load (which would wait on the
@@ -384,16 +412,23 @@ __global__ __launch_bounds__(kMfmaThreads<R>, kMfmaPerCu<R>) void k_tile_spread_
                 R nf0 = nd.f[0], nf1 = nd.f[1], nf2 = nd.f[2], fre = fv.x, fim = fv.y;
                 asm volatile("" : "+v"(loc), "+v"(nf0), "+v"(nf1), "+v"(nf2), "+v"(fre), "+v"(fim));
                 const int lo0 = loc & 255, lo1 = (loc >> 8) & 255, loL = (loc >> 16) & 255;
-                const bool s1 = S::SETS2 && valid && lo0 > S::LO_MAX0;
+                // the node's sets (DUP: possibly both)
+                const bool in1 = S::SETS2 && valid && lo0 > S::LO_MAX0;
+                const bool in0 = valid && (!in1 || (S::DUP && lo0 < S::OFF1));
                 // set masks over the lower half; rank = the node's place in its set
-                const uint64_t m1 = __ballot(s1 && half == 0), m0 = __ballot(valid && !s1 && half == 0);
+                const uint64_t m1 = __ballot(in1 && half == 0), m0 = __ballot(in0 && half == 0);
                 const int n0 = __popcll(m0), n1 = __popcll(m1);
                 const int p0pad = (n0 + 3) & ~3, npos = p0pad + ((n1 + 3) & ~3);
-                const uint64_t mine = s1 ? m1 : m0;
-                const int rank = __popcll(mine & ((1ull << nl) - 1ull));
-                const int pos = s1 ? p0pad + rank : rank;
+                const uint64_t below = (1ull << nl) - 1ull;
                 if (wave < 3 * PW) {
-                    if (valid) {
+#pragma unroll 1
+                    for (int set = 0; set < (S::DUP ? 2 : 1); ++set) {
+                        // one pass over the nodes, or (DUP) one per set
+                        if (S::DUP ? !(set ? in1 : in0) : !valid) continue;
+                        const bool s1 = S::DUP ? set == 1 : in1;
+                        const int pos = s1 ? p0pad + __popcll(m1 & below) : __popcll(m0 & below);
+                        // a node of both sets has its planes below 16 in set 0
+                        const int x_min = S::DUP && s1 && in0 && wave / PW == 0 ? 16 - S::OFF1 : 0;
                         const int t = PW == 1 ? wave : wave / PW;   // axis
                         const int tq = PW == 1 ? half : PW * half + (wave - t * PW);
                         const R ft = t == 0 ? nf0 : (t == 1 ? nf1 : nf2);
@@ -427,7 +462,7 @@ __global__ __launch_bounds__(kMfmaThreads<R>, kMfmaPerCu<R>) void k_tile_spread_
                                 else if constexpr (WIN == WIN_KAISER_BESSEL) w = kb_phi<R>(sv, (R)wc.m, shpt);
                                 else if constexpr (WIN == WIN_SINC) w = sinc_phi<R>(sv, wc.m, shpt);
                                 else w = nrt * wexp<R>(-kbt * sv * sv);
-                                v[u] = l >= 0 && l < W ? w : (R)0;
+                                v[u] = l >= 0 && l < W && (!S::DUP || x0 + u >= x_min) ? w : (R)0;
                             }
 #pragma unroll
                             for (int u = 0; u < 4; ++u) row[x0 + u] = v[u] * sc0;
@@ -448,87 +483,138 @@ __global__ __launch_bounds__(kMfmaThreads<R>, kMfmaPerCu<R>) void k_tile_spread_
                     }
                 }
                 __syncthreads();
-                // the next batch of this chunk loads during this one's steps
-                if (s0 + S::NB < ch.count) {
-                    const uint32_t sn = s0 + S::NB + (uint32_t)nl;
-                    if (sn < ch.count) {
-                        nd = desc[ch.start + sn];
-                        fv = fs[ch.start + sn];
+                // the next batch of this chunk, or the first one of the next chunk,
+                // loads during this one's steps
+                {
+                    const bool more = s0 + S::NB < ch.count;
+                    const uint32_t sn = (more ? s0 + S::NB : 0u) + (uint32_t)nl;
+                    const uint32_t at = (more ? ch.start : chn.start) + sn;
+                    if (sn < (more ? ch.count : cn < n ? chn.count : 0u)) {
+                        nd = desc[at];
+                        fv = fs[at];
                     }
                 }
                 ksteps(p0pad >> 2, S::SETS2 ? npos >> 2 : p0pad >> 2);
             }
-            // the sum of the two sets per plane into the slot image; register i of lane
-            // group g holds plane M::row(g, i) of set 0 and M::row(g, i) + OFF1 of set 1
-            auto put = [&](const acc_t &v0, const acc_t &v1, int b, int cl, bool ok) {
-                R up[4];   // set 1 at plane M::row(g, i)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if (!S::SETS2) {
-                        up[i] = (R)0;
-                    } else if constexpr (sizeof(R) == 4) {
-                        // plane 4g + i of set 1 is row 4g + i - OFF1: this lane
-                        // group's register i - OFF1, or the previous group's
-                        if (i >= S::OFF1) {
-                            up[i] = v1[i - S::OFF1];
-                        } else {
-                            const R t = __shfl(v1[4 - S::OFF1 + i], lane - 16);
-                            up[i] = g > 0 ? t : (R)0;
-                        }
-                    } else {
-                        // plane g + 4i of set 1 is row g - OFF1 + 4i: register i of lane
-                        // group g - OFF1, or register i - 1 of group g - OFF1 + 4
-                        const R t1 = __shfl(v1[i], lane - 16 * S::OFF1);
-                        const R t2 = i > 0 ? __shfl(v1[i > 0 ? i - 1 : 0], lane + 16 * (4 - S::OFF1)) : (R)0;
-                        up[i] = g >= S::OFF1 ? t1 : t2;
-                    }
-                }
-                if (!ok) return;
-                if constexpr (sizeof(R) == 4) {
-                    const MfmaSlotCol o = mfma_slot_col<L>(g, b, cl, ri);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (4 * g + i < S::P) stg[o.base + i * o.step] = v0[i] + up[i];
-                    if (S::SETS2 && g == 3) {
-#pragma unroll
-                        for (int i = 0; i < S::OFF1; ++i) stg[o.base16 + i * o.step] = v1[4 - S::OFF1 + i];
-                    }
-                } else {
+            // What the next chunk leaves of the accumulators: all of them (the same
+            // tile), the columns [8, 16) as its [0, 8) (the next tile of the row), or none.
+            const bool seg_end = ((c + 1) & segm) == 0 || c + 1 >= n;
+            const bool same = !seg_end && chn.tile == ch.tile;
+            const bool chain = !seg_end && chn.tile == ch.tile + 1 && chn.tile % ntl != 0;
+            const uint32_t cur_c = c;
+            if (!same) {
+                // the lane's place anew for every image, opaque to the compiler: its
+                // image offsets, invariant over the chunks, would else be kept in
+                // registers through the matrix steps (or spilled there)
+                int ln = lane;
+                asm volatile("" : "+v"(ln));
+                const int g = (ln >> 4) & 3, ri = ln & 1, cc = (ln & 15) >> 1;
+                // the sum of the two sets per plane into the slot image (its part from
+                // cell `from` on); register i of lane group g holds plane M::row(g, i) of
+                // set 0 and M::row(g, i) + OFF1 of set 1
+                auto put = [&](const acc_t &v0, const acc_t &v1, int b, int cl, bool ok, int from) {
+                    R up[4];   // set 1 at plane M::row(g, i)
+                    constexpr int OFF1 = S::OFF1;
+                    // floor(x / 4) for x >= -8
+                    auto fl4 = [](int x) constexpr { return (x + 8) / 4 - 2; };
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const int a = g + 4 * i;
-                        if (a < S::P) stg[mfma_slot_off<L>(a, b, cl, ri)] = v0[i] + up[i];
+                        if constexpr (!S::SETS2) {
+                            up[i] = (R)0;
+                        } else if constexpr (sizeof(R) == 4) {
+                            // plane 4g + i is row 4g + i - OFF1 of set 1: register rg of the
+                            // lane group dg before this one
+                            const int dg = -fl4(i - OFF1), rg = i - OFF1 + 4 * dg;
+                            if (dg == 0) {
+                                up[i] = v1[rg];
+                            } else {
+                                const R t = __shfl(v1[rg], ln - 16 * dg);
+                                up[i] = g >= dg ? t : (R)0;
+                            }
+                        } else {
+                            // plane g + 4i is row g - OFF1 + 4i of set 1: lane group
+                            // (g - OFF1) mod 4, register i - K there, or i - K + 1 where
+                            // g - OFF1 reaches one more multiple of 4
+                            constexpr int K = (OFF1 + 3) / 4;
+                            const int src = (((g - OFF1) & 3) << 4) | (ln & 15);
+                            const R t1 = i - K + 1 >= 0 ? __shfl(v1[i - K + 1 > 0 ? i - K + 1 : 0], src) : (R)0;
+                            const R t2 = i - K >= 0 ? __shfl(v1[i - K > 0 ? i - K : 0], src) : (R)0;
+                            up[i] = g >= OFF1 - 4 * (K - 1) ? t1 : t2;
+                        }
                     }
-                    // planes 16 + j (rows 16 - OFF1 + j of set 1: register 3 of group 4 - OFF1 + j)
-                    if (S::SETS2 && g >= 4 - S::OFF1)
-                        stg[mfma_slot_off<L>(16 + g - (4 - S::OFF1), b, cl, ri)] = v1[3];
+                    if (!ok) return;
+                    if constexpr (sizeof(R) == 4) {
+                        // four planes of one block, and those from 16 on
+                        const int EL = L::ext(L::TL, L::PL, cl >> 3), E1 = L::ext(L::T1, L::P1, b >> 3);
+                        const int step = 2 * E1 * EL;
+                        const int o = mfma_slot_off<L>(4 * g, b, cl, ri, from);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (4 * g + i < S::P) stg[o + i * step] = v0[i] + up[i];
+                        if constexpr (S::SETS2) {
+                            const int o16 = mfma_slot_off<L>(16, b, cl, ri, from);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const int a = 4 * g + i + OFF1;
+                                if (a >= 16) stg[o16 + (a - 16) * step] = v1[i];
+                            }
+                        }
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int a = g + 4 * i;
+                            if (a < S::P) stg[mfma_slot_off<L>(a, b, cl, ri, from)] = v0[i] + up[i];
+                        }
+                        if constexpr (S::SETS2) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const int a = g + 4 * i + OFF1;
+                                if (a >= 16) stg[mfma_slot_off<L>(a, b, cl, ri, from)] = v1[i];
+                            }
+                        }
+                    }
+                };
+                V16 *dst = reinterpret_cast<V16 *>(slots + (int64_t)cur_c * L::SC);
+                const V16 *src = reinterpret_cast<const V16 *>(stg);
+                constexpr int N1 = 2 * CS::HALF1 / E16, NS = 2 * L::SC / E16;
+                if (!chain) {
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) {
+                        put(acc0[r][1], acc1[r][1], rb + r, 8 + cc, 8 + cc < S::P, 0);
+                        acc0[r][1] = acc1[r][1] = z4;
+                    }
+                    if constexpr (!ONE) {
+                        __syncthreads();
+                        for (int i = tid; i < N1; i += NT) stream_store(dst + i, src[i]);
+                        __syncthreads();   // the image is free again
+                    }
                 }
-            };
 #pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                put(acc0[r][0], acc1[r][0], rb + r, cc, cc < S::P);
-                put(acc0[r][1], acc1[r][1], rb + r, 8 + cc, 8 + cc < S::P);
+                for (int r = 0; r < NR; ++r) {
+                    put(acc0[r][0], acc1[r][0], rb + r, cc, true, FROM0);
+                    acc0[r][0] = acc0[r][1];
+                    acc1[r][0] = acc1[r][1];
+                    acc0[r][1] = acc1[r][1] = z4;
+                }
+#pragma unroll
+                for (int j = 0; j < NL; ++j) {
+                    put(accL0[j], accL1[j], lb_b[j], lb_c[j], lb_ok[j], FROM0);
+                    accL0[j] = accL1[j] = z4;
+                }
+                if (seg_end && tid == 0) s_tk[0] = ticket;
+                __syncthreads();   // the image is whole and the ticket visible
+                busy = false;
+                // the next chunk writes the image only after its first batch's barrier,
+                // which every wavefront reaches after its copy-out reads
+                const int i0 = ONE && !chain ? 0 : N1;
+                for (int i = i0 + tid; i < NS; i += NT) stream_store(dst + i, src[ONE ? i : i - N1]);
             }
-#pragma unroll
-            for (int j = 0; j < NL; ++j) put(accL0[j], accL1[j], lb_b[j], lb_c[j], lb_ok[j]);
-            if (tid == 0) s_tk[0] = ticket;
-            __syncthreads();   // the image is whole and the ticket visible
-            const uint32_t cur_c = c;
+            if (seg_end) nxt = first_chunk(ticket_at(0));
             c = cn;
             ch = chn;
-            cn = s_tk[0];
-            // the next chunk's first batch loads during the copy-out, and the record
-            // of the chunk after it during the next chunk's steps
-            if (c < n && (uint32_t)nl < ch.count) {
-                nd = desc[ch.start + nl];
-                fv = fs[ch.start + nl];
-            }
+            cn = after(c);
+            // the record of the chunk after the next loads during the next one's steps
             if (cn < n) chn = chunks[cn];
-            // the next chunk writes the image only after its first batch's barrier,
-            // which every wavefront reaches after its copy-out reads
-            V16 *dst = reinterpret_cast<V16 *>(slots + (int64_t)cur_c * L::SC);
-            const V16 *src = reinterpret_cast<const V16 *>(stg);
-            for (int i = tid; i < 2 * L::SC / E16; i += NT) stream_store(dst + i, src[i]);
         }
     };
 

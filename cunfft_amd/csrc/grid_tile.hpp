@@ -187,6 +187,63 @@ template <typename T, int D, int W, int PS, int V> struct TileLayout {
     }
 };
 
+// Slot of the matrix-core spread's chains (grid_mfma.hpp): the blocks of
+// TileLayout::block_off ordered by their place along the last axis, [8, 16) first
+// (HALF1 cells, written at the end of a chain only), then [0, 8) and the rest
+// (written for every tile), so both parts are contiguous.
+//
+// A chain is up to 2^seg_shift consecutive chunks (a segment: chunk index >>
+// seg_shift) of one tile or of neighbours along the last axis.  Of a tile's chunks
+// c0 .. cl the last one and each last one of a segment write their slot, the others
+// nothing; the [8, 16) part of cl is not written when the chain goes on into the next
+// tile of the row.
+template <typename L> struct ChainSlot {
+    static constexpr int HALF1 = (L::P0 * L::P1 * L::ext(L::TL, L::PL, 1) + L::CPL - 1) / L::CPL * L::CPL;
+    static_assert(L::QL >= 2 && L::QL <= 3, "");
+    static constexpr int first(int qL)
+    {
+        return qL == 1 ? 0 : HALF1 + (qL == 2 ? L::P0 * L::P1 * L::TL : 0);
+    }
+    static constexpr int off(int q0, int q1, int qL)
+    {
+        return first(qL) + L::ext(L::TL, L::PL, qL) * (q0 * L::T0 * L::P1 + L::ext(L::T0, L::P0, q0) * q1 * L::T1);
+    }
+    static_assert(HALF1 + L::P0 * L::P1 * (L::PL - L::ext(L::TL, L::PL, 1)) <= L::SC, "the slot holds both parts");
+};
+
+// The slots with a sum of one tile's block qL: count of them, and the chunk of the
+// k-th.  CH false: every chunk of the tile.
+template <bool CH> struct SlotList {
+    uint32_t c0, n, last;
+    int sh;
+    // c0: the tile's first chunk, nc its chunk count; goes_on: qL is 1 and the tile
+    // after it in the row (with the tile to fold) has nodes
+    __host__ __device__ __forceinline__ SlotList(uint32_t c0_, uint32_t nc, bool goes_on, int shift)
+    {
+        c0 = c0_;
+        n = nc;
+        last = 0;
+        sh = 0;
+        if constexpr (CH) {
+            sh = shift;
+            last = c0_ + nc - 1u;
+            c0 = c0_ >> sh;
+            if (nc > 0) n = (last >> sh) - c0 + 1u;
+            if (goes_on && nc > 0 && ((last + 1u) & ((1u << sh) - 1u)) != 0) --n;
+        }
+    }
+    __host__ __device__ __forceinline__ SlotList() {}
+    __host__ __device__ __forceinline__ uint32_t at(uint32_t k) const
+    {
+        if constexpr (CH) {
+            const uint32_t e = ((c0 + k + 1u) << sh) - 1u;
+            return e < last ? e : last;
+        } else {
+            return c0 + k;
+        }
+    }
+};
+
 // ----------------------------------------------------------- helpers ----
 
 // The Kaiser-Bessel and sinc weights out of line: the Gaussian path keeps its
@@ -489,6 +546,13 @@ template <typename T> __device__ __forceinline__ void kahan_add(T &s, T &e, T x)
     const T t = s + y;
     e = (t - s) - y;
     s = t;
+}
+
+// Cell offset of a block in a slot of the plain or of the chains' order.
+template <typename L, bool CH> constexpr int slot_block(int q0, int q1, int qL)
+{
+    if constexpr (CH) return ChainSlot<L>::off(q0, q1, qL);
+    else return L::block_off(q0, q1, qL);
 }
 
 // Fold sum: plain, or Neumaier's compensated sum (c collects the low parts;
@@ -1561,7 +1625,7 @@ __global__ __launch_bounds__(256) void k_sorted_coeffs_batch(const GridJob<T> *_
 // candidate tiles of one leading-axis offset is loaded at once (a dense tile's
 // further chunks follow), and the sums run in a fixed order: the result does
 // not depend on scheduling.
-template <typename T, int D, int W, int PS, int V, bool COMP>
+template <typename T, int D, int W, int PS, int V, bool COMP, bool CH>
 __device__ __forceinline__ void tile_fold(const cplx_t<T> *__restrict__ slots,
                                           const uint32_t *__restrict__ tile_count,
                                           const uint32_t *__restrict__ chunk_start,
@@ -1598,10 +1662,11 @@ __device__ __forceinline__ void tile_fold(const cplx_t<T> *__restrict__ slots,
     for (int k = 0; k < CPT; ++k) sx[k] = sy[k] = 0;
 #pragma unroll
     for (int q0 = 0; q0 < L::Q0; ++q0) {
-        uint32_t c0[QR], nch[QR];
+        SlotList<CH> sl[QR];
         int li[QR][CPT];
         bool ok[QR][CPT];
         C v[QR][CPT];
+        uint32_t row_nc = 0;
 #pragma unroll
         for (int qq = 0; qq < QR; ++qq) {
             const int q1 = qq / L::QL, qL = qq % L::QL;
@@ -1613,10 +1678,11 @@ __device__ __forceinline__ void tile_fold(const cplx_t<T> *__restrict__ slots,
                 const uint32_t ntt = (uint32_t)bg.nt[t];
                 src = src * ntt + (tk[t] + ntt * 4 - (uint32_t)qv[t]) % ntt;
             }
-            const uint32_t cnt = tile_count[src];
-            c0[qq] = chunk_start[src];
-            nch[qq] = chunks_of(cnt, bg.chunk_base);
-            const int boff = L::block_off(q0, q1, qL);
+            const uint32_t nc = chunks_of(tile_count[src], bg.chunk_base);
+            if (qL == 0) row_nc = nc;   // the chunks of the row's tile at this tile's place
+            sl[qq] = SlotList<CH>(chunk_start[src], nc, qL == 1 && row_nc > 0 && tk[D - 1] > 0, bg.seg_shift);
+            const uint32_t cnt = sl[qq].n;
+            const int boff = slot_block<L, CH>(q0, q1, qL);
 #pragma unroll
             for (int k = 0; k < CPT; ++k) {
                 ok[qq][k] = cnt > 0 && slice0 + threadIdx.x + 256 * k < CORE && r0[k] < E0 &&
@@ -1629,7 +1695,7 @@ __device__ __forceinline__ void tile_fold(const cplx_t<T> *__restrict__ slots,
 #pragma unroll
             for (int k = 0; k < CPT; ++k) {
                 // a candidate with no nodes reads chunk 0 and adds nothing
-                const C *sp = slots + (int64_t)(ok[qq][k] ? c0[qq] : 0) * L::SC;
+                const C *sp = slots + (int64_t)(ok[qq][k] ? sl[qq].at(0) : 0) * L::SC;
                 v[qq][k] = sp[ok[qq][k] ? li[qq][k] : 0];
             }
 #pragma unroll
@@ -1643,12 +1709,12 @@ __device__ __forceinline__ void tile_fold(const cplx_t<T> *__restrict__ slots,
         // further chunks of dense candidate tiles, four loads in flight
 #pragma unroll
         for (int qq = 0; qq < QR; ++qq)
-            for (uint32_t c = 1; c < nch[qq]; c += 4) {
+            for (uint32_t c = 1; c < sl[qq].n; c += 4) {
                 C w[4][CPT];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    const bool in = c + u < nch[qq];
-                    const C *sp = slots + (int64_t)(in ? c0[qq] + c + u : 0) * L::SC;
+                    const bool in = c + u < sl[qq].n;
+                    const C *sp = slots + (int64_t)(in ? sl[qq].at(c + u) : 0) * L::SC;
 #pragma unroll
                     for (int k = 0; k < CPT; ++k) w[u][k] = sp[ok[qq][k] && in ? li[qq][k] : 0];
                 }
@@ -1656,7 +1722,7 @@ __device__ __forceinline__ void tile_fold(const cplx_t<T> *__restrict__ slots,
                 for (int u = 0; u < 4; ++u)
 #pragma unroll
                     for (int k = 0; k < CPT; ++k)
-                        if (ok[qq][k] && c + u < nch[qq]) {
+                        if (ok[qq][k] && c + u < sl[qq].n) {
                             fold_add<COMP>(sx[k], cx[k], w[u][k].x);
                             fold_add<COMP>(sy[k], cy[k], w[u][k].y);
                         }
@@ -1722,7 +1788,7 @@ template <typename L> struct Fold3Shape {
                   "column segments tile the core and whole workgroups");
 };
 
-template <typename T, int D, int W, int PS, int V, bool COMP>
+template <typename T, int D, int W, int PS, int V, bool COMP, bool CH>
 __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slots,
                                                const uint32_t *__restrict__ tile_count,
                                                const uint32_t *__restrict__ chunk_start,
@@ -1763,19 +1829,22 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
     const uint32_t n0 = (uint32_t)bg.nt[0], n1 = D == 3 ? (uint32_t)bg.nt[1] : 1u,
                    n2 = (uint32_t)bg.nt[D - 1];
     constexpr int Q0 = L::Q0, Q1 = L::Q1, QL = L::QL;
-    // first chunk and chunk count of the candidate tile q back along each axis
-    uint32_t c0[Q0][Q1][QL], nch[Q0][Q1][QL];
+    // slots of the candidate tile q back along each axis
+    SlotList<CH> sl[Q0][Q1][QL];
 #pragma unroll
     for (int q0 = 0; q0 < Q0; ++q0)
 #pragma unroll
-        for (int q1 = 0; q1 < Q1; ++q1)
+        for (int q1 = 0; q1 < Q1; ++q1) {
+            uint32_t row_nc = 0;
 #pragma unroll
             for (int qL = 0; qL < QL; ++qL) {
                 const uint32_t src = ((tk[0] + 4 * n0 - q0) % n0 * n1 + (tk[1] + 4 * n1 - q1) % n1) * n2 +
                                      (tk[2] + 4 * n2 - qL) % n2;
-                c0[q0][q1][qL] = chunk_start[src];
-                nch[q0][q1][qL] = chunks_of(tile_count[src], bg.chunk_base);
+                const uint32_t nc = chunks_of(tile_count[src], bg.chunk_base);
+                if (qL == 0) row_nc = nc;   // the chunks of the row's tile at this tile's place
+                sl[q0][q1][qL] = SlotList<CH>(chunk_start[src], nc, qL == 1 && row_nc > 0 && tk[2] > 0, bg.seg_shift);
             }
+        }
     T sx[SEGC], sy[SEGC], cx[SEGC], cy[SEGC];
 #pragma unroll
     for (int i = 0; i < SEGC; ++i) sx[i] = sy[i] = cx[i] = cy[i] = 0;
@@ -1807,16 +1876,17 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
 #pragma unroll
             for (int qL = 0; qL < QL; ++qL) {
                 // a candidate with no nodes reads chunk 0 and adds nothing
-                const C *sp = slots + (int64_t)(nch[q0][q1][qL] > 0 ? c0[q0][q1][qL] : 0) * L::SC;
+                const SlotList<CH> &sq = sl[q0][q1][qL];
+                const C *sp = slots + (int64_t)(sq.n > 0 ? sq.at(0) : 0) * L::SC;
                 const int EL = L::ext(TL, L::PL, qL);
-                const int o = L::block_off(q0, q1, qL) + rc * EL;
+                const int o = slot_block<L, CH>(q0, q1, qL) + rc * EL;
                 if (EL == TL) load_full(sp, o + seg * SEGC, v[qL]);
                 else load_last(sp, o, v[qL]);
             }
 #pragma unroll
             for (int qL = 0; qL < QL; ++qL) {
                 const int EL = L::ext(TL, L::PL, qL);
-                const bool ok = nch[q0][q1][qL] > 0 && in01;
+                const bool ok = sl[q0][q1][qL].n > 0 && in01;
 #pragma unroll
                 for (int i = 0; i < SEGC; ++i)
                     if ((EL == TL || (i < NLAST && seg * SEGC + i < EL)) && ok) {
@@ -1828,27 +1898,31 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
 #pragma unroll
             for (int qL = 0; qL < QL; ++qL) {
                 const int EL = L::ext(TL, L::PL, qL);
-                const int o = L::block_off(q0, q1, qL) + rc * EL;
-                const uint32_t nc = nch[q0][q1][qL];
-                for (uint32_t c = 1; c < nc; c += 4) {
-                    C w[4][SEGC];
+                const int o = slot_block<L, CH>(q0, q1, qL) + rc * EL;
+                const SlotList<CH> &sq = sl[q0][q1][qL];
+                const uint32_t nc = sq.n;
+                uint32_t c = 1;
+                auto slot_group = [&](auto n_c) {   // the next n_c slots, their loads together
+                    constexpr int NC = decltype(n_c)::value;
+                    C w[NC][SEGC];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        // past the last chunk: the last one again, not added
-                        const uint32_t cu = c + u < nc ? c + u : nc - 1;
-                        const C *sp = slots + (int64_t)(c0[q0][q1][qL] + cu) * L::SC;
+                    for (int u = 0; u < NC; ++u) {
+                        const C *sp = slots + (int64_t)sq.at(c + u) * L::SC;
                         if (EL == TL) load_full(sp, o + seg * SEGC, w[u]);
                         else load_last(sp, o, w[u]);
                     }
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
+                    for (int u = 0; u < NC; ++u)
 #pragma unroll
                         for (int i = 0; i < SEGC; ++i)
-                            if ((EL == TL || (i < NLAST && seg * SEGC + i < EL)) && in01 && c + u < nc) {
+                            if ((EL == TL || (i < NLAST && seg * SEGC + i < EL)) && in01) {
                                 fold_add<COMP>(sx[i], cx[i], w[u][i].x);
                                 fold_add<COMP>(sy[i], cy[i], w[u][i].y);
                             }
-                }
+                    c += NC;
+                };
+                while (c + 4 <= nc) slot_group(std::integral_constant<int, 4>{});
+                while (c < nc) slot_group(std::integral_constant<int, 1>{});
             }
         }
     const uint32_t g1 = D == 3 ? (uint32_t)ge.n[1] : 1u, gL = (uint32_t)ge.n[D - 1];
@@ -1859,16 +1933,16 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
                    cmake<T>(sx[2 * i + 1] + cx[2 * i + 1], sy[2 * i + 1] + cy[2 * i + 1]));
 }
 
-template <typename T, int D, int W, int PS, int V, bool COMP>
+template <typename T, int D, int W, int PS, int V, bool COMP, bool CH>
 __global__ __launch_bounds__(256) void k_tile_fold(const cplx_t<T> *__restrict__ slots,
                                                    const uint32_t *__restrict__ tile_count,
                                                    const uint32_t *__restrict__ chunk_start,
                                                    cplx_t<T> *__restrict__ g, Geom ge, BinGeom bg)
 {
     if constexpr (kFoldColumns<T, D>)
-        tile_fold_cols<T, D, W, PS, V, COMP>(slots, tile_count, chunk_start, g, ge, bg, blockIdx.x);
+        tile_fold_cols<T, D, W, PS, V, COMP, CH>(slots, tile_count, chunk_start, g, ge, bg, blockIdx.x);
     else
-        tile_fold<T, D, W, PS, V, COMP>(slots, tile_count, chunk_start, g, ge, bg, blockIdx.x,
+        tile_fold<T, D, W, PS, V, COMP, CH>(slots, tile_count, chunk_start, g, ge, bg, blockIdx.x,
                                         blockIdx.y);
 }
 
@@ -1883,9 +1957,9 @@ __global__ __launch_bounds__(256) void k_tile_fold_batch(const GridJob<T> *__res
     const BlockMap bm = map[blockIdx.x];
     const GridJob<T> &J = jobs[bm.job];
     if constexpr (kFoldColumns<T, D>)
-        tile_fold_cols<T, D, W, PS, V, false>(J.slots, J.tile_count, J.chunk_start, J.g, J.ge, J.bg, bm.blk);
+        tile_fold_cols<T, D, W, PS, V, false, false>(J.slots, J.tile_count, J.chunk_start, J.g, J.ge, J.bg, bm.blk);
     else
-        tile_fold<T, D, W, PS, V, false>(J.slots, J.tile_count, J.chunk_start, J.g, J.ge, J.bg,
+        tile_fold<T, D, W, PS, V, false, false>(J.slots, J.tile_count, J.chunk_start, J.g, J.ge, J.bg,
                                          bm.blk / SLICES, (int)(bm.blk % SLICES));
 }
 
@@ -2113,7 +2187,7 @@ template <typename T> struct SpreadOp {
                         static_cast<const NodeDesc<T> *>(b.desc), fs, b.chunks, b.n_chunks, slots,
                         win_const<T>(ge));
                     if (mid) CUNFFT_HIP(hipEventRecord(mid, s));
-                    k_tile_fold<T, D, W, NWS, V, true><<<fold_grid, 256, 0, s>>>(
+                    k_tile_fold<T, D, W, NWS, V, true, false><<<fold_grid, 256, 0, s>>>(
                         slots, b.tile_count, b.chunk_start, g, ge, bin_geom(b));
                     return true;
                 }
@@ -2126,9 +2200,10 @@ template <typename T> struct SpreadOp {
                                                       : k_tile_spread_mfma<T, W, WIN_GAUSSIAN>;
                 constexpr int NT = MfmaSpread<T, W>::NW * 64;
                 k_clear_u32<<<1, 64, 0, s>>>(b.n_chunks + 1);
-                const unsigned grid = (unsigned)std::min<int64_t>(b.max_chunks, resident_blocks(km, NT));
+                const int64_t segs = (b.max_chunks >> b.seg_shift) + 1;
+                const unsigned grid = (unsigned)std::min<int64_t>(segs, resident_blocks(km, NT));
                 km<<<grid, NT, 0, s>>>(static_cast<const NodeDesc<T> *>(b.desc), fs, b.chunks, b.n_chunks, slots,
-                                       win_const<T>(ge));
+                                       win_const<T>(ge), b.seg_shift, (uint32_t)b.nt[2]);
             } else if constexpr (MFMA2) {
                 k_tile_spread_mfma2<W><<<(unsigned)b.max_chunks, 64, 0, s>>>(
                     reinterpret_cast<const NodeDesc<float> *>(b.desc), reinterpret_cast<const cplx_t<float> *>(fs),
@@ -2149,7 +2224,7 @@ template <typename T> struct SpreadOp {
                     win_const<T>(ge));
             }
             if (mid) CUNFFT_HIP(hipEventRecord(mid, s));
-            k_tile_fold<T, D, W, NWS, V, false><<<fold_grid, 256, 0, s>>>(
+            k_tile_fold<T, D, W, NWS, V, false, MFMA><<<fold_grid, 256, 0, s>>>(
                 slots, b.tile_count, b.chunk_start, g, ge, bin_geom(b));
             return true;
         } else {

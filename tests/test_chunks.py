@@ -2,8 +2,8 @@
 
 Compiled for the host from cunfft_amd/csrc/bin.hpp:
 
-* ``chunk_shift`` / ``chunks_of``: a tile's chunks hold 2^base .. 256 nodes, at
-  most kTileChunksAim of them until they are 256 long, and never more than
+* ``chunk_shift`` / ``chunks_of``: a tile's chunks hold 2^base .. 256 nodes, fewer
+  than 1 << kTileChunksLog of them until they are 256 long, and never more than
   c / 2^base rounded up, so a binning's ntiles + ceil(M / 2^base) chunk records
   suffice;
 * ``xcd_chunk`` with ``xcd_group``: every chunk exactly once within the workgroups
@@ -33,8 +33,8 @@ int main()
             bad += !(s >= base && s <= kChunkShift);
             bad += !(k * (uint64_t)len >= c && (k == 0 ? c == 0 : (k - 1) * (uint64_t)len < c));
             bad += !(k <= (c + (1u << base) - 1) >> base);
-            bad += !(s == kChunkShift || c >> s <= (uint32_t)kTileChunksAim);
-            bad += !(s == base || c >> (s - 1) > (uint32_t)kTileChunksAim);   // no longer than needed
+            bad += !(s == kChunkShift || c >> s < 1u << kTileChunksLog);
+            bad += !(s == base || c >> (s - 1) >= 1u << kTileChunksLog);   // no longer than needed
         }
     printf("chunks %d\n", bad);
     bad = 0;

@@ -400,9 +400,11 @@ __global__ __launch_bounds__(kTileBlock) void k_bin_chunks(const uint32_t *__res
 // Hence about 1024 chunks at most from splitting in 2D, and 128 nodes or more in 3D,
 // whose slots are larger: there only where no evenly filled tile is split (at 123 nodes
 // per tile, where a third would be, 342 us instead of 293).  A batch has its problems
-// to fill the GPU: the longest chunks.
+// to fill the GPU: the longest chunks.  1D, one wavefront per chunk and node per lane:
+// 64 nodes a chunk while that is at most 512 chunks.
 static int plan_chunk_base(int d, int64_t M, int64_t ntiles)
 {
+    if (d == 1) return M <= 32768 ? 6 : M <= 65536 ? 7 : kChunkShift;
     if (d == 3) return M <= 80 * ntiles && (M >> 7) <= 4096 ? 7 : kChunkShift;
     int s = kChunkShiftMin;
     while (s < kChunkShift && (M >> s) > 1024) ++s;
@@ -451,7 +453,7 @@ bool Binning::plan(const Geom &ge, int elem_bytes_, int kernel_variant, int tile
         if (t < d) bytes *= T[t] + W - 1;
     }
     if (ntiles >= (int64_t(1) << 31)) return false;
-    chunk_base = planes() && own_scratch ? plan_chunk_base(d, ge.M, ntiles) : kChunkShift;
+    chunk_base = own_scratch && (planes() || d == 1) ? plan_chunk_base(d, ge.M, ntiles) : kChunkShift;
     seg_shift = planes() && own_scratch ? plan_seg_shift(elem_bytes, ntiles) : 0;
     if (planes()) {
         // plane-tiled kernels: 32-bit grid offsets and the LDS tile must fit

@@ -114,11 +114,13 @@ template <> struct alignas(16) NodeDesc<double> {
 struct BinGeom;
 
 // Nodes sorted on the device by the grid tile that holds the start of their
-// window, u_t mod n_t, and -- for the plane-tiled kernels -- within a tile by
-// their window start there: row and column unit first, plane last (sub_key),
+// window, u_t mod n_t, and -- where the 3D VALU spread takes them -- within a
+// tile by their window start there: row and column unit first, plane last (sub_key),
 // so nodes whose windows cover the same rows and column units follow each
 // other with rising plane (the adjoint accumulates such a run in registers
-// and writes the tile once per run).  The sort is a stable LSD radix sort of
+// and writes the tile once per run).  The other kernels take a tile's nodes in any
+// order, and the key without its 8 to 10 low bits sorts in one radix pass less (two
+// in 2D on up to 256 tiles).  The sort is a stable LSD radix sort of
 // the composite key tile * sub_range + sub_key over the node indices, so
 // nodes with equal keys keep their index order: the sorted order, and with
 // it the order of every adjoint sum, depends on the nodes only, never on
@@ -139,6 +141,7 @@ struct Binning {
     int64_t nt[3] = {1, 1, 1};  // tiles per axis
     int64_t ntiles = 0;
     int64_t M = 0;
+    bool sub_sort = true;       // nodes sorted within their tile by sub_key (else by index)
     int chunk_base = kChunkShift;   // log2 of the nodes per chunk (chunk_shift)
     int seg_shift = 0;          // log2 of the chunks per chain of the matrix-core spread
     int64_t max_chunks = 0;
@@ -190,6 +193,7 @@ struct BinGeom {
     int64_t nt[3];
     int64_t ntiles;
     int sub_shift;   // column cells per lane unit, log2 (FP32 1, FP64 0)
+    int sub_sort;    // nodes sorted within their tile by sub_key (else by index)
     int chunk_base;  // log2 of the nodes per chunk (chunk_shift)
     int seg_shift;   // log2 of the chunks per chain (ChainSlot)
 };
@@ -207,6 +211,7 @@ __host__ __device__ inline uint32_t sub_key(int d, const uint32_t (&lo)[3], cons
 }
 inline uint32_t sub_range(const BinGeom &g)
 {
+    if (!g.sub_sort) return 1;
     uint32_t r = (1u << g.logT[0]) * ((1u << g.logT[g.d - 1]) >> g.sub_shift);
     return g.d == 3 ? r << g.logT[1] : r;
 }

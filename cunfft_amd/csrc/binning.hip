@@ -43,6 +43,7 @@ BinGeom bin_geom(const Binning &b)
     }
     g.ntiles = b.ntiles;
     g.sub_shift = b.elem_bytes == 4 ? 1 : 0;
+    g.sub_sort = b.sub_sort;
     g.chunk_base = b.chunk_base;
     g.seg_shift = b.seg_shift;
     return g;
@@ -468,9 +469,12 @@ bool Binning::plan(const Geom &ge, int elem_bytes_, int kernel_variant, int tile
         if (d == 3 && W > 14) return false;
     }
     // the composite sort key must fit 32 bits
-    const uint64_t sr = planes() ? sub_range(bin_geom(*this)) : 1u;
-    const uint64_t kmax = (uint64_t)ntiles * sr;
-    if (kmax > (uint64_t(1) << 32)) return false;
+    sub_sort = true;
+    if (planes() && (uint64_t)ntiles * sub_range(bin_geom(*this)) > (uint64_t(1) << 32)) return false;
+    // a run of nodes is only kept in registers by the 3D VALU spread: not on the matrix
+    // cores (8^3 tiles, W <= 14, a plan's own binning; a batch's 3D spread is the VALU's)
+    sub_sort = d == 3 && !(tile_variant == 0 && W <= 14 && own_scratch);
+    const uint64_t kmax = (uint64_t)ntiles * (planes() ? sub_range(bin_geom(*this)) : 1u);
     int bits = 1;
     while ((uint64_t(1) << bits) < kmax) ++bits;
     key_bits = bits;

@@ -82,7 +82,8 @@ template <> __device__ __forceinline__ double win_exp<double>(double v) { return
 // The weights of a node batch are one evaluation per lane on the way to every
 // gridding loop, and the library's sinh and sin are long.  Here: Taylor sums up to
 // z = 1, above it one exponential for both hyperbolic functions, and sin and cos from
-// one reduction by multiples of pi (z <= 2 pi sqrt(2m+1) < 26 for a node's taps).
+// one reduction by multiples of pi (a node's taps have |s| <= m + 3/2, so z is at most
+// 2 pi sqrt(3m + 9/4) there: 33 for m <= 8, 45 for m = 16).
 // Nodes set, forward and adjoint of 50021 2D nodes, m = 3, FP32: 171 -> 146 us; ten
 // CGNR iterations over 100800 2D nodes, m = 4, FP64: 5.2 -> 3.85 ms (with the
 // chunk rule of binning.hip).
@@ -100,16 +101,28 @@ template <typename T> __device__ __forceinline__ T kb_series(T q)
     return p;
 }
 
-// exp(z) for 0 < z <= kKbZMax.  FP32: the hardware exp2 of the rounded z log2(e),
-// times what the rounding left.
-__device__ __forceinline__ float kb_exp(float z)
+// sinh(z) / z for 1 < z <= b m (b < 2 pi, m <= 16: below 101).  FP32: the hardware
+// exp2 of the rounded z log2(e), times what the rounding left.
+//  * exp(z) leaves the FP32 range at z = 88.7, where sinh(z) / z does not yet (m = 15
+//    and 16 at an oversampling of 4.5 and more get there), so it is taken at an eighth:
+//    hi - 3 is exact for hi >= 1.44 (and must not be contracted with the product, of
+//    which lo is the rest).
+//  * log2(e) is rounded down for hi, so lo is positive and what is past the range is
+//    infinite, not NaN.
+__device__ __forceinline__ float kb_sinhc(float z)
 {
-    const float hi = z * 1.44269504f;
-    const float lo = fmaf(z, 1.44269504f, -hi) + z * 1.92596299e-8f;   // log2(e) in two parts
-    const float e = __builtin_amdgcn_exp2f(hi);
-    return fmaf(e, lo * 0.693147181f, e);
+#pragma clang fp contract(off)
+    const float hi = z * 1.44269490f;
+    const float lo = fmaf(z, 1.92596299e-8f, fmaf(z, 1.44269504f, -hi));   // log2(e) in two parts
+    const float x = __builtin_amdgcn_exp2f(hi - 3.f);
+    const float e = fmaf(x, lo * 0.693147181f, x);
+    return 4.f * (e - 0x1p-6f / e) / z;
 }
-__device__ __forceinline__ double kb_exp(double z) { return exp(z); }
+__device__ __forceinline__ double kb_sinhc(double z)
+{
+    const double e = exp(z);
+    return 0.5 * (e - 1.0 / e) / z;
+}
 
 __device__ __forceinline__ float kb_reduce(float z, float k)   // z - k pi, pi in two parts
 {
@@ -146,8 +159,7 @@ template <typename T> __device__ __forceinline__ T kb_phi(T s, T m, T b)
     } else if (!(z <= (T)kKbZMax)) {
         v = z * (T)0;
     } else if (d > (T)0) {
-        const T e = kb_exp(z);
-        v = (T)0.5 * (e - (T)1 / e) / z;
+        v = kb_sinhc(z);
     } else {
         T c;
         kb_sincos<T>(z, v, c);
@@ -201,7 +213,7 @@ template <> __device__ __forceinline__ double kb_dphi<double>(double s, double m
     } else if (!(z <= (T)kKbZMax)) {
         v = z * (T)0;
     } else if (d > (T)0) {
-        const T e = kb_exp(z), i = (T)1 / e;
+        const T e = exp(z), i = (T)1 / e;
         v = ((T)0.5 * (e + i) - (T)0.5 * (e - i) / z) / (z * z);
     } else {
         T sn, cs;

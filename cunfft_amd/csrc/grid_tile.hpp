@@ -1894,7 +1894,11 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
                         fold_add<COMP>(sy[i], cy[i], v[qL][i].y);
                     }
             }
-            // further chunks of dense candidate tiles, four loads in flight
+            // further chunks of dense candidate tiles, four loads in flight.  Not for the
+            // compensated sums of the widest 3D windows: with four, the loops over their
+            // candidates are too long to be unrolled and the table of slots goes to
+            // scratch memory (m = 5, 5001 nodes on a 128^3 grid: fold 101 us, with one 41).
+            constexpr bool FOUR = !(COMP && D == 3 && W >= 12);
 #pragma unroll
             for (int qL = 0; qL < QL; ++qL) {
                 const int EL = L::ext(TL, L::PL, qL);
@@ -1921,7 +1925,8 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
                             }
                     c += NC;
                 };
-                while (c + 4 <= nc) slot_group(std::integral_constant<int, 4>{});
+                if constexpr (FOUR)
+                    while (c + 4 <= nc) slot_group(std::integral_constant<int, 4>{});
                 while (c < nc) slot_group(std::integral_constant<int, 1>{});
             }
         }

@@ -19,17 +19,34 @@
 #include <hip/amd_detail/amd_hip_unsafe_atomics.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "bin.hpp"
 
 namespace cunfft {
 
-// Threads per workgroup.  A 1D tile is 4 KB and holds about 128 nodes at one node per
-// coefficient, so one wavefront per chunk keeps its lanes busy, needs no other to
-// stage or flush the tile, and 32 of them fit a CU; the tiles of d >= 2 fill most of a
-// CU's LDS.  1D, n = 2^23, 2^22 nodes, m = 4, FP64: gather 190 -> 127 us, scatter with
-// its clears 230 -> 146 us (also by the cells it stores instead of adding).
-template <int D> constexpr int kTileThreads = D == 1 ? 64 : 256;
+// Threads per workgroup: 256, and 64 where a 1D launch has very many chunks.  A 1D tile
+// is 4 KB, so 32 one-wavefront workgroups fit a CU, and none of a chunk's wavefronts
+// waits for another to stage or flush the tile; but a wavefront alone takes a chunk's 256
+// nodes 64 after 64, so it needs enough workgroups beside it and few nodes per tile.
+// Forward / adjoint in us, 64 against 256 threads (m = 4):
+//   FP64, 32768 tiles of 128 nodes   gather 127 / 190, scatter with its clears 146 / 230
+//   FP64, 8192 tiles   48 nodes a tile 53 / 55, 60 / 78    200 nodes 75 / 73, 84 / 91
+//   FP64, 2048 tiles   48 nodes        32 / 32, 35 / 37   1000 nodes 64 / 63, 101 / 88
+//   FP64,  512 tiles  200 nodes        26 / 21, 29 / 24   1000 nodes 35 / 31, 43 / 37
+//   FP64,    4 tiles 4000 nodes        15 / 11, 18 / 14   (FP32 the same, smaller)
+//   FP64,    8 tiles 125000 nodes      30 / 31, 87 / 99   32 tiles 33000 nodes 40 / 40, 79 / 82
+// Hence 64 for plans from 2048 tiles on with at most 256 nodes each, and for the sums of
+// very many chunks (2^19 nodes) into few tiles (2^15 nodes each).  A batch deals the
+// chunks of all its jobs: 64 from 8192 chunks on (36900 chunks of 256 nodes FP32 94 / 111,
+// 198 / 229; 8192 of 80 nodes 53 / 55, 70 / 77; 48 chunks 18 / 17, 23 / 21).
+constexpr int kTileThreads = 256, kTileThreadsNarrow = 64;
+static bool narrow_groups(const Binning &b)
+{
+    if (b.d != 1) return false;
+    return b.ntiles >= 2048 ? b.M <= 256 * b.ntiles : b.M >= (int64_t(1) << 19) && b.M >= b.ntiles << 15;
+}
+static bool narrow_groups(int d, uint32_t batch_chunks) { return d == 1 && batch_chunks >= 8192; }
 constexpr int kMaxTileBytes = 120 * 1024;
 
 template <int D, int W> struct Pad {
@@ -96,7 +113,7 @@ __device__ __forceinline__ int node_local(const double *__restrict__ xs, uint32_
 }
 
 // --------------------------------------------------------- tiled gather --
-template <typename T, int D, int W>
+template <typename T, int D, int W, int NT>
 __device__ __forceinline__ void gather_tiled(const cplx_t<T> *__restrict__ g,
                                              const double *__restrict__ xs,
                                              const uint32_t *__restrict__ perm, const Chunk ch,
@@ -104,7 +121,6 @@ __device__ __forceinline__ void gather_tiled(const cplx_t<T> *__restrict__ g,
                                              const BinGeom &bg)
 {
     using PD = Pad<D, W>;
-    constexpr int NT = kTileThreads<D>;
     __shared__ cplx_t<T> tile[PD::PT];
     int64_t o[3];
     tile_origin<D>(ch.tile, bg, o);
@@ -172,23 +188,23 @@ __device__ __forceinline__ void gather_tiled(const cplx_t<T> *__restrict__ g,
     }
 }
 
-template <typename T, int D, int W>
-__global__ __launch_bounds__(kTileThreads<D>) void k_gather_tiled(
+template <typename T, int D, int W, int NT>
+__global__ __launch_bounds__(NT) void k_gather_tiled(
     const cplx_t<T> *__restrict__ g, const double *__restrict__ xs, const uint32_t *__restrict__ perm,
     const Chunk *__restrict__ chunks, const uint32_t *__restrict__ n_chunks, cplx_t<T> *__restrict__ f,
     Geom ge, BinGeom bg)
 {
     if (blockIdx.x >= n_chunks[0]) return;
-    gather_tiled<T, D, W>(g, xs, perm, chunks[blockIdx.x], f, ge, bg);
+    gather_tiled<T, D, W, NT>(g, xs, perm, chunks[blockIdx.x], f, ge, bg);
 }
 
-template <typename T, int D, int W>
-__global__ __launch_bounds__(kTileThreads<D>) void k_gather_tiled_batch(
+template <typename T, int D, int W, int NT>
+__global__ __launch_bounds__(NT) void k_gather_tiled_batch(
     const GridJob<T> *__restrict__ jobs, const BlockMap *__restrict__ map)
 {
     const BlockMap bm = map[blockIdx.x];
     const GridJob<T> &J = jobs[bm.job];
-    gather_tiled<T, D, W>(J.g, J.xs, J.perm, J.chunks[bm.blk], J.f_out, J.ge, J.bg);
+    gather_tiled<T, D, W, NT>(J.g, J.xs, J.perm, J.chunks[bm.blk], J.f_out, J.ge, J.bg);
 }
 
 // -------------------------------------------------------- tiled scatter --
@@ -198,7 +214,7 @@ __device__ __forceinline__ void lds_add(T *p, T v)
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-template <typename T, typename A, int D, int W>
+template <typename T, typename A, int D, int W, int NT>
 __device__ __forceinline__ void scatter_tiled(const double *__restrict__ xs,
                                               const uint32_t *__restrict__ perm,
                                               const cplx_t<T> *__restrict__ f, const Chunk ch,
@@ -206,7 +222,6 @@ __device__ __forceinline__ void scatter_tiled(const double *__restrict__ xs,
                                               const BinGeom &bg, bool own = false)
 {
     using PD = Pad<D, W>;
-    constexpr int NT = kTileThreads<D>;
     __shared__ A acc_re[PD::PT];
     __shared__ A acc_im[PD::PT];
     int64_t o[3];
@@ -269,15 +284,15 @@ __device__ __forceinline__ void scatter_tiled(const double *__restrict__ xs,
     }
 }
 
-template <typename T, typename A, int D, int W>
-__global__ __launch_bounds__(kTileThreads<D>) void k_scatter_tiled(
+template <typename T, typename A, int D, int W, int NT>
+__global__ __launch_bounds__(NT) void k_scatter_tiled(
     const double *__restrict__ xs, const uint32_t *__restrict__ perm, const cplx_t<T> *__restrict__ f,
     const Chunk *__restrict__ chunks, const uint32_t *__restrict__ n_chunks,
     const uint32_t *__restrict__ tile_count, cplx_t<T> *__restrict__ g, Geom ge, BinGeom bg)
 {
     if (blockIdx.x >= n_chunks[0]) return;
     const Chunk ch = chunks[blockIdx.x];
-    scatter_tiled<T, A, D, W>(xs, perm, f, ch, g, ge, bg,
+    scatter_tiled<T, A, D, W, NT>(xs, perm, f, ch, g, ge, bg,
                               D == 1 && chunks_of(tile_count[ch.tile], bg.chunk_base) == 1);
 }
 
@@ -294,13 +309,13 @@ __global__ __launch_bounds__(256) void k_zero_shared(const uint32_t *__restrict_
     for (int i = threadIdx.x & 63; i < n; i += 64) g[tile * TileShape<1>::T[0] + i] = cmake<T>(0, 0);
 }
 
-template <typename T, typename A, int D, int W>
-__global__ __launch_bounds__(kTileThreads<D>) void k_scatter_tiled_batch(
+template <typename T, typename A, int D, int W, int NT>
+__global__ __launch_bounds__(NT) void k_scatter_tiled_batch(
     const GridJob<T> *__restrict__ jobs, const BlockMap *__restrict__ map)
 {
     const BlockMap bm = map[blockIdx.x];
     const GridJob<T> &J = jobs[bm.job];
-    scatter_tiled<T, A, D, W>(J.xs, J.perm, J.f_in, J.chunks[bm.blk], J.g, J.ge, J.bg);
+    scatter_tiled<T, A, D, W, NT>(J.xs, J.perm, J.f_in, J.chunks[bm.blk], J.g, J.ge, J.bg);
 }
 
 // Grid <- 0 for the node-lane scatter of every job, 1024 cells per block.
@@ -317,13 +332,25 @@ __global__ __launch_bounds__(256) void k_zero_batch(const GridJob<T> *__restrict
 }
 
 // ------------------------------------------------------------ dispatch --
+// go(threads per workgroup), the number as a constant
+template <int D, typename F> static void lane_launch(bool narrow, F &go)
+{
+    if constexpr (D == 1)
+        if (narrow) return go(std::integral_constant<int, kTileThreadsNarrow>{});
+    go(std::integral_constant<int, kTileThreads>{});
+}
+
 template <typename T, int D, int W>
 static void launch_gather_lanes(const Geom &ge, const Binning &b, const cplx_t<T> *g, cplx_t<T> *f,
                                 hipStream_t s)
 {
     if constexpr (tile_fits<T, D, W>()) {
-        k_gather_tiled<T, D, W><<<(unsigned)b.max_chunks, kTileThreads<D>, 0, s>>>(
-            g, b.xs, b.perm, b.chunks, b.n_chunks, f, ge, bin_geom(b));
+        auto go = [&](auto nt) {
+            constexpr int NT = decltype(nt)::value;
+            k_gather_tiled<T, D, W, NT><<<(unsigned)b.max_chunks, NT, 0, s>>>(
+                g, b.xs, b.perm, b.chunks, b.n_chunks, f, ge, bin_geom(b));
+        };
+        lane_launch<D>(narrow_groups(b), go);
     } else {
         throw Error(CUNFFT_ERR_UNSUPPORTED, "tile does not fit in LDS");
     }
@@ -338,8 +365,12 @@ static void launch_scatter_lanes(const Geom &ge, const Binning &b, const cplx_t<
             k_zero_shared<T, W><<<(unsigned)((b.ntiles + 3) / 4), 256, 0, s>>>(b.tile_count, bin_geom(b), g);
         else
             launch_zero<T>(g, ge.n[0] * ge.n[1] * ge.n[2], s);
-        k_scatter_tiled<T, double, D, W><<<(unsigned)b.max_chunks, kTileThreads<D>, 0, s>>>(
-            b.xs, b.perm, f, b.chunks, b.n_chunks, b.tile_count, g, ge, bin_geom(b));
+        auto go = [&](auto nt) {
+            constexpr int NT = decltype(nt)::value;
+            k_scatter_tiled<T, double, D, W, NT><<<(unsigned)b.max_chunks, NT, 0, s>>>(
+                b.xs, b.perm, f, b.chunks, b.n_chunks, b.tile_count, g, ge, bin_geom(b));
+        };
+        lane_launch<D>(narrow_groups(b), go);
     } else {
         throw Error(CUNFFT_ERR_UNSUPPORTED, "tile does not fit in LDS");
     }
@@ -423,10 +454,14 @@ static void launch_lanes_batch(BatchStage st, const GridJob<T> *jobs, const Bloc
                                uint32_t nblk, hipStream_t s)
 {
     if constexpr (tile_fits<T, D, W>()) {
-        if (st == BS_GATHER)
-            k_gather_tiled_batch<T, D, W><<<nblk, kTileThreads<D>, 0, s>>>(jobs, map);
-        else
-            k_scatter_tiled_batch<T, double, D, W><<<nblk, kTileThreads<D>, 0, s>>>(jobs, map);
+        auto go = [&](auto nt) {
+            constexpr int NT = decltype(nt)::value;
+            if (st == BS_GATHER)
+                k_gather_tiled_batch<T, D, W, NT><<<nblk, NT, 0, s>>>(jobs, map);
+            else
+                k_scatter_tiled_batch<T, double, D, W, NT><<<nblk, NT, 0, s>>>(jobs, map);
+        };
+        lane_launch<D>(narrow_groups(D, nblk), go);
     } else {
         throw Error(CUNFFT_ERR_UNSUPPORTED, "tile does not fit in LDS");
     }

@@ -401,8 +401,8 @@ __global__ __launch_bounds__(kTileBlock) void k_bin_chunks(const uint32_t *__res
 // Hence about 1024 chunks at most from splitting in 2D, and 128 nodes or more in 3D,
 // whose slots are larger: there only where no evenly filled tile is split (at 123 nodes
 // per tile, where a third would be, 342 us instead of 293).  A batch has its problems
-// to fill the GPU: the longest chunks.  1D, one wavefront per chunk and node per lane:
-// 64 nodes a chunk while that is at most 512 chunks.
+// to fill the GPU: the longest chunks.  1D, a node per lane: 64 nodes a chunk while that
+// is at most 512 chunks.
 static int plan_chunk_base(int d, int64_t M, int64_t ntiles)
 {
     if (d == 1) return M <= 32768 ? 6 : M <= 65536 ? 7 : kChunkShift;

@@ -13,7 +13,7 @@
 // Twiddles come from a per-length table computed in extended precision on the
 // host.
 //
-// The usual line lengths (8 .. 4096 powers of two, 3 2^k and 9 2^k up to 1536)
+// The usual line lengths (4 .. 4096 powers of two, 3 2^k and 9 2^k from 48 to 1536)
 // run the register-resident pass of fft_line.hpp.  This file holds the set-up
 // of the passes and the generic pass for the other lengths 2^a 3^b: each
 // workgroup loads C whole lines into LDS, runs Stockham stages there and writes

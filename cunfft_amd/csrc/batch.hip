@@ -60,6 +60,7 @@ template <typename T> struct BatchImpl {
         size_t pass_off = 0;           // into passes (FFT stages)
         size_t lds = 0;
         bool fft_line = false;         // register-resident passes (FFT stages)
+        int threads = 64;              // per workgroup of such a launch
     };
 
     int d = 0, m = 0, W = 0, R = 0;
@@ -328,6 +329,7 @@ template <typename T> struct BatchImpl {
                         ph.push_back(f.P);
                         for (int64_t k = 0; k < f.blocks; ++k) mh.push_back(BlockMap{job, (uint32_t)k});
                         L.lds = std::max(L.lds, f.lds);
+                        L.threads = std::max(L.threads, (f.P.C * f.P.tpl + 63) / 64 * 64);
                     }
                 }
                 L.nblk = (uint32_t)(mh.size() - L.map_off);
@@ -384,7 +386,7 @@ template <typename T> struct BatchImpl {
         for (const Launch &L : stages[dir]) {
             if (L.fft_t >= 0 && L.fft_line)
                 launch_fft_line_batch<T>(passes + L.pass_off, maps + L.map_off, L.nblk, L.fft_t == d - 1,
-                                         L.lds, s);
+                                         L.threads, L.lds, s);
             else if (L.fft_t >= 0)
                 launch_fft_batch<T>(passes + L.pass_off, maps + L.map_off, L.nblk, L.lds, s);
             else

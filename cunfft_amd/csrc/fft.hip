@@ -481,8 +481,8 @@ static int line_pitch_of(int L)
 // points on, where 256 threads hold too few adjacent columns), columns at most
 // one 128-byte line wide.  A small grid takes fewer lines per workgroup, down to
 // one wavefront (rows) or 64 bytes of a row (columns), until 512 workgroups
-// spread over the 256 CUs.  A batch launches 256-thread workgroups for all its
-// jobs, which are many: always full ones.
+// spread over the 256 CUs.  A batch's jobs are many and share a launch of at most 256
+// threads per workgroup: always the full number of lines.
 //
 // Generic pass: rows are packed up to 2048 elements per workgroup; strided
 // passes take adjacent columns up to kFftElems elements.

@@ -532,8 +532,11 @@ __global__ __launch_bounds__(line_threads_max<L>(), (line_waves<T, LinePlan<L>::
     fft_line<T, L, MAPI, MAPO, SPLIT>(P, blk, reinterpret_cast<cplx_t<T> *>(line_lds));
 }
 
-// The passes of many transforms in one grid of 256-thread workgroups (the
-// jobs' lengths differ; LDS sized for the largest).  Rows and columns apart.
+// The passes of many transforms in one grid (the jobs' lengths differ; threads, 256 at
+// most, and LDS for the largest workgroup among them).  Rows and columns apart.  Short
+// lines need few threads, and idle wavefronts would hold the registers of others: six
+// 3D problems of 64^3 grids x 2, FP64, 497 -> 309 us (forward), 256 x 8 lines of 1024
+// points FP32 53 -> 36 us against 256 threads for all.
 template <typename T, int MAP>
 __global__ __launch_bounds__(256, (line_waves<T, 24>())) void k_fft_line_batch(const FftPass<T> *__restrict__ passes,
                                                         const BlockMap *__restrict__ map)
@@ -589,10 +592,10 @@ template <typename T> void launch_fft_line(const FftPass<T> &P, int64_t blocks, 
 
 template <typename T>
 void launch_fft_line_batch(const FftPass<T> *passes, const BlockMap *map, uint32_t nblk, bool rows,
-                           size_t lds, hipStream_t s)
+                           int threads, size_t lds, hipStream_t s)
 {
-    if (rows) k_fft_line_batch<T, MAP_ROWS><<<nblk, 256, lds, s>>>(passes, map);
-    else k_fft_line_batch<T, MAP_COLS><<<nblk, 256, lds, s>>>(passes, map);
+    if (rows) k_fft_line_batch<T, MAP_ROWS><<<nblk, threads, lds, s>>>(passes, map);
+    else k_fft_line_batch<T, MAP_COLS><<<nblk, threads, lds, s>>>(passes, map);
     CUNFFT_HIP(hipGetLastError());
 }
 

@@ -136,7 +136,7 @@ void launch_fft_line(const FftPass<T> &p, int64_t blocks, size_t lds_bytes, hipS
 // launch shape.  tw is the twiddle table of length n_t.  Axes longer than
 // kFftMaxLine need fft_axis_setup.
 // What a pass is set up for: a transform of its own, a batch's launch over many
-// (256-thread workgroups), or the grid of an FP32 node gradient.  The gradient is
+// (256 threads per workgroup at most), or the grid of an FP32 node gradient.  The gradient is
 // handed out as float64 values (autograd.py), so its bits are kept: the mixed
 // line lengths, whose radices the register-resident pass orders differently, run
 // the generic pass there (the power-of-two lines give the same bits in both).
@@ -167,13 +167,13 @@ struct BlockMap {
 };
 // One launch of the passes of many transforms (one FftPass per job): generic
 // passes, or register-resident ones set up for a batch (rows: along the last
-// axis).
+// axis; threads: the widest workgroup's, a multiple of 64).
 template <typename T>
 void launch_fft_batch(const FftPass<T> *passes, const BlockMap *map, uint32_t nblk,
                       size_t lds_bytes, hipStream_t s);
 template <typename T>
 void launch_fft_line_batch(const FftPass<T> *passes, const BlockMap *map, uint32_t nblk, bool rows,
-                           size_t lds_bytes, hipStream_t s);
+                           int threads, size_t lds_bytes, hipStream_t s);
 
 // ------------------------------------------------------------ gridding ---
 template <typename T>

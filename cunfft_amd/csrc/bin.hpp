@@ -23,6 +23,25 @@ __host__ __device__ __forceinline__ uint32_t chunks_of(uint32_t c, int base)
     const int s = chunk_shift(c, base);
     return (c + (1u << s) - 1u) >> s;
 }
+// log2 of the chunks per chain of the 3D matrix-core spread (and its fold), for the n
+// chunks that M nodes came to; seg_shift: the most, by the plan (plan_seg_shift).  A
+// chain saves slots between neighbouring tiles and between the chunks of one tile, and
+// costs the fold a table of its slots per tile.  With few chunks, or few tiles holding
+// nodes, there is nothing to save, and a chain only makes work of several workgroups the
+// work of one.  Adjoint in us, chains / single chunks (m = 4):
+//   FP64 128^3 grid, uniform    100 nodes 96 / 70, 1000 108 / 100, 20001 171 / 179
+//   FP64 256^3 grid, uniform   1000 nodes 565 / 391, 3000 602 / 502, 20001 820 / 839
+//   FP64 one point,  20001 nodes in 79 chunks: 128^3 155 / 107, 256^3 657 / 322
+//   a tenth of each axis, 100001 nodes: 128^3 FP64 181 / 244, FP32 135 / 155;
+//     192 x 192 x 96 FP64 205 / 241; 256^3 FP64 574 / 478, FP32 288 / 266
+//   FP32 128^3 grid, uniform    100 nodes 55 / 49, 3000 83 / 86, 20001 99 / 117
+// So chains from a chunk per CU on, where they are an eighth of the tiles, or a 32nd if
+// they are full (64 nodes and more: many chunks per tile).
+__host__ __device__ __forceinline__ int chain_shift(uint32_t n, uint32_t M, uint32_t ntiles, int seg_shift)
+{
+    const bool pays = n >= ntiles / 8 || (M / 64 >= n && n >= ntiles / 32);
+    return n >= 256u && pays ? seg_shift : 0;
+}
 constexpr int kFoldSegBytes = 32;   // bytes of a core column one fold thread sums (FP32, d >= 2)
 
 // Grid tile per dimension: the nodes whose window starts in one tile are

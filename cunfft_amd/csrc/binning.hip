@@ -412,7 +412,8 @@ static int plan_chunk_base(int d, int64_t M, int64_t ntiles)
     return s;
 }
 
-// log2 of the chunks per chain of the 3D matrix-core spread.  A chain of k tiles writes
+// log2 of the chunks per chain of the 3D matrix-core spread, at most (chain_shift, by the
+// chunks there are, may take none).  A chain of k tiles writes
 // (9 k + 8) / (17 k) of the slots that single chunks write (W = 10) and is one
 // workgroup's work in one piece.  Forward + adjoint (the adjoint at m = 6) in us for
 // chains of 1 / 2 / 4 / 8 chunks:

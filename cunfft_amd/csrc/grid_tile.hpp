@@ -548,10 +548,11 @@ template <typename T> __device__ __forceinline__ void kahan_add(T &s, T &e, T x)
     s = t;
 }
 
-// Cell offset of a block in a slot of the plain or of the chains' order.
-template <typename L, bool CH> constexpr int slot_block(int q0, int q1, int qL)
+// Cell offset of a block in a slot of the plain or of the chains' order (CS; CH, below:
+// the slots are those of chains).
+template <typename L, bool CS> constexpr int slot_block(int q0, int q1, int qL)
 {
-    if constexpr (CH) return ChainSlot<L>::off(q0, q1, qL);
+    if constexpr (CS) return ChainSlot<L>::off(q0, q1, qL);
     else return L::block_off(q0, q1, qL);
 }
 
@@ -1625,7 +1626,7 @@ __global__ __launch_bounds__(256) void k_sorted_coeffs_batch(const GridJob<T> *_
 // candidate tiles of one leading-axis offset is loaded at once (a dense tile's
 // further chunks follow), and the sums run in a fixed order: the result does
 // not depend on scheduling.
-template <typename T, int D, int W, int PS, int V, bool COMP, bool CH>
+template <typename T, int D, int W, int PS, int V, bool COMP, bool CS, bool CH, bool SPARSE>
 __device__ __forceinline__ void tile_fold(const cplx_t<T> *__restrict__ slots,
                                           const uint32_t *__restrict__ tile_count,
                                           const uint32_t *__restrict__ chunk_start,
@@ -1682,13 +1683,22 @@ __device__ __forceinline__ void tile_fold(const cplx_t<T> *__restrict__ slots,
             if (qL == 0) row_nc = nc;   // the chunks of the row's tile at this tile's place
             sl[qq] = SlotList<CH>(chunk_start[src], nc, qL == 1 && row_nc > 0 && tk[D - 1] > 0, bg.seg_shift);
             const uint32_t cnt = sl[qq].n;
-            const int boff = slot_block<L, CH>(q0, q1, qL);
+            const int boff = slot_block<L, CS>(q0, q1, qL);
 #pragma unroll
             for (int k = 0; k < CPT; ++k) {
                 ok[qq][k] = cnt > 0 && slice0 + threadIdx.x + 256 * k < CORE && r0[k] < E0 &&
                             r1[k] < E1 && rL[k] < EL;
                 li[qq][k] = boff + (r0[k] * E1 + r1[k]) * EL + rL[k];
             }
+        }
+        if constexpr (SPARSE) {
+            // nothing from this offset along the leading axis: nothing to load (where most
+            // tiles hold nodes the branch costs more than it saves: it keeps the loads of
+            // one offset from passing the sums of the one before)
+            uint32_t any = 0;
+#pragma unroll
+            for (int qq = 0; qq < QR; ++qq) any |= sl[qq].n;
+            if (any == 0) continue;
         }
 #pragma unroll
         for (int qq = 0; qq < QR; ++qq)
@@ -1788,7 +1798,7 @@ template <typename L> struct Fold3Shape {
                   "column segments tile the core and whole workgroups");
 };
 
-template <typename T, int D, int W, int PS, int V, bool COMP, bool CH>
+template <typename T, int D, int W, int PS, int V, bool COMP, bool CS, bool CH>
 __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slots,
                                                const uint32_t *__restrict__ tile_count,
                                                const uint32_t *__restrict__ chunk_start,
@@ -1879,7 +1889,7 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
                 const SlotList<CH> &sq = sl[q0][q1][qL];
                 const C *sp = slots + (int64_t)(sq.n > 0 ? sq.at(0) : 0) * L::SC;
                 const int EL = L::ext(TL, L::PL, qL);
-                const int o = slot_block<L, CH>(q0, q1, qL) + rc * EL;
+                const int o = slot_block<L, CS>(q0, q1, qL) + rc * EL;
                 if (EL == TL) load_full(sp, o + seg * SEGC, v[qL]);
                 else load_last(sp, o, v[qL]);
             }
@@ -1902,7 +1912,7 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
 #pragma unroll
             for (int qL = 0; qL < QL; ++qL) {
                 const int EL = L::ext(TL, L::PL, qL);
-                const int o = slot_block<L, CH>(q0, q1, qL) + rc * EL;
+                const int o = slot_block<L, CS>(q0, q1, qL) + rc * EL;
                 const SlotList<CH> &sq = sl[q0][q1][qL];
                 const uint32_t nc = sq.n;
                 uint32_t c = 1;
@@ -1938,17 +1948,32 @@ __device__ __forceinline__ void tile_fold_cols(const cplx_t<T> *__restrict__ slo
                    cmake<T>(sx[2 * i + 1] + cx[2 * i + 1], sy[2 * i + 1] + cy[2 * i + 1]));
 }
 
-template <typename T, int D, int W, int PS, int V, bool COMP, bool CH>
+template <typename T, int D, int W, int PS, int V, bool COMP, bool CS>
 __global__ __launch_bounds__(256) void k_tile_fold(const cplx_t<T> *__restrict__ slots,
                                                    const uint32_t *__restrict__ tile_count,
                                                    const uint32_t *__restrict__ chunk_start,
+                                                   const uint32_t *__restrict__ n_chunks,
                                                    cplx_t<T> *__restrict__ g, Geom ge, BinGeom bg)
 {
-    if constexpr (kFoldColumns<T, D>)
-        tile_fold_cols<T, D, W, PS, V, COMP, CH>(slots, tile_count, chunk_start, g, ge, bg, blockIdx.x);
-    else
-        tile_fold<T, D, W, PS, V, COMP, CH>(slots, tile_count, chunk_start, g, ge, bg, blockIdx.x,
-                                        blockIdx.y);
+    auto fold = [&](auto ch, auto sparse) {
+        constexpr bool CH = decltype(ch)::value, SPARSE = decltype(sparse)::value;
+        if constexpr (kFoldColumns<T, D>)
+            tile_fold_cols<T, D, W, PS, V, COMP, CS, CH>(slots, tile_count, chunk_start, g, ge, bg, blockIdx.x);
+        else
+            tile_fold<T, D, W, PS, V, COMP, CS, CH, SPARSE>(slots, tile_count, chunk_start, g, ge, bg,
+                                                            blockIdx.x, blockIdx.y);
+    };
+    using std::false_type;
+    using std::true_type;
+    if constexpr (CS) {
+        const uint32_t n = n_chunks[0], nt = (uint32_t)bg.ntiles;
+        if (chain_shift(n, (uint32_t)ge.M, nt, bg.seg_shift) > 0) return fold(true_type{}, false_type{});
+        // few tiles with nodes (FP64, 256^3 grid, adjoint of 1000 nodes 491 -> 391 us, of
+        // 20001 at one point 468 -> 322)
+        if constexpr (!kFoldColumns<T, D>)
+            if (n < nt / 8) return fold(false_type{}, true_type{});
+    }
+    fold(false_type{}, false_type{});
 }
 
 // Batched fold: block blk of a job is tile blk / slices, slice blk % slices.
@@ -1962,9 +1987,9 @@ __global__ __launch_bounds__(256) void k_tile_fold_batch(const GridJob<T> *__res
     const BlockMap bm = map[blockIdx.x];
     const GridJob<T> &J = jobs[bm.job];
     if constexpr (kFoldColumns<T, D>)
-        tile_fold_cols<T, D, W, PS, V, false, false>(J.slots, J.tile_count, J.chunk_start, J.g, J.ge, J.bg, bm.blk);
+        tile_fold_cols<T, D, W, PS, V, false, false, false>(J.slots, J.tile_count, J.chunk_start, J.g, J.ge, J.bg, bm.blk);
     else
-        tile_fold<T, D, W, PS, V, false, false>(J.slots, J.tile_count, J.chunk_start, J.g, J.ge, J.bg,
+        tile_fold<T, D, W, PS, V, false, false, false, false>(J.slots, J.tile_count, J.chunk_start, J.g, J.ge, J.bg,
                                          bm.blk / SLICES, (int)(bm.blk % SLICES));
 }
 
@@ -2193,7 +2218,7 @@ template <typename T> struct SpreadOp {
                         win_const<T>(ge));
                     if (mid) CUNFFT_HIP(hipEventRecord(mid, s));
                     k_tile_fold<T, D, W, NWS, V, true, false><<<fold_grid, 256, 0, s>>>(
-                        slots, b.tile_count, b.chunk_start, g, ge, bin_geom(b));
+                        slots, b.tile_count, b.chunk_start, b.n_chunks, g, ge, bin_geom(b));
                     return true;
                 }
             }
@@ -2208,7 +2233,8 @@ template <typename T> struct SpreadOp {
                 const int64_t segs = (b.max_chunks >> b.seg_shift) + 1;
                 const unsigned grid = (unsigned)std::min<int64_t>(segs, resident_blocks(km, NT));
                 km<<<grid, NT, 0, s>>>(static_cast<const NodeDesc<T> *>(b.desc), fs, b.chunks, b.n_chunks, slots,
-                                       win_const<T>(ge), b.seg_shift, (uint32_t)b.nt[2]);
+                                       win_const<T>(ge), b.seg_shift, (uint32_t)ge.M, (uint32_t)b.ntiles,
+                                       (uint32_t)b.nt[2]);
             } else if constexpr (MFMA2) {
                 k_tile_spread_mfma2<W><<<(unsigned)b.max_chunks, 64, 0, s>>>(
                     reinterpret_cast<const NodeDesc<float> *>(b.desc), reinterpret_cast<const cplx_t<float> *>(fs),
@@ -2230,7 +2256,7 @@ template <typename T> struct SpreadOp {
             }
             if (mid) CUNFFT_HIP(hipEventRecord(mid, s));
             k_tile_fold<T, D, W, NWS, V, false, MFMA><<<fold_grid, 256, 0, s>>>(
-                slots, b.tile_count, b.chunk_start, g, ge, bin_geom(b));
+                slots, b.tile_count, b.chunk_start, b.n_chunks, g, ge, bin_geom(b));
             return true;
         } else {
             return false;

@@ -39,7 +39,7 @@ __host__ __device__ __forceinline__ int sign_bit(double x) { return __builtin_si
 // n - 1, src/cunfft_kernel.cu:528-531, which needs a power of two).
 // wrap_hi: a in [0, 2n) (a wrapped window start plus a tap offset < n).
 __device__ __forceinline__ int64_t wrap_hi(int64_t a, int64_t n) { return a >= n ? a - n : a; }
-__device__ __forceinline__ uint32_t wrap_hi32(uint32_t a, uint32_t n) { return a >= n ? a - n : a; }
+__host__ __device__ __forceinline__ uint32_t wrap_hi32(uint32_t a, uint32_t n) { return a >= n ? a - n : a; }
 
 // Floor modulo a mod n in [0, n) for any a; the division runs only outside
 // [-n, n), i.e. for nodes outside [-1/2, 1/2).

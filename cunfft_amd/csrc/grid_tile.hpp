@@ -569,6 +569,18 @@ template <bool COMP, typename T> __device__ __forceinline__ void fold_add(T &s, 
     }
 }
 
+// Grid column from which unit un of a padded row that starts at column o is staged.  The
+// used cells of a row wrap once; the spare units behind them (up to the pitch; no node
+// reads them) could reach past a second copy of the shortest axis (8 columns at W = 8,
+// 16 at W = 14 and 16 of the 16^2 tiles, FP32), and so past the grid's end: where the
+// pitch allows that they are staged from the row's first column.
+template <typename L> __host__ __device__ __forceinline__ uint32_t stage_column(uint32_t o, int un, uint32_t nL)
+{
+    constexpr int W = L::PL - L::TL + 1, SHORTEST = (W + L::TL - 1) / L::TL * L::TL;
+    const int c = L::CPL * un;
+    return wrap_hi32(o + (L::RP - L::TL > SHORTEST && c >= L::RL ? 0 : c), nL);
+}
+
 // Stages the halo-padded grid tile `tile_id` into LDS (rows of the pitch,
 // 16 bytes per load, every padded row wrapped onto the grid).  rowoff_mem is
 // LDS scratch for the padded rows' grid offsets (used when they fit in
@@ -620,7 +632,7 @@ __device__ __forceinline__ void stage_tile(const cplx_t<T> *__restrict__ g, uint
         __syncthreads();
     }
     const int un = tid % NR, r0 = tid / NR;
-    const uint32_t colc = wrap_hi32(o[D - 1] + CPL * un, nL);
+    const uint32_t colc = stage_column<L>(o[D - 1], un, nL);
     if (r0 < RS) {
         for (int rb = r0; rb < ROWS; rb += SB * RS) {
             VT v[SB];

@@ -102,6 +102,18 @@ template <typename R, int W> struct MfmaSpread {
     static constexpr int NB = 32;                       // nodes per batch
     // batch rows: each set padded to 4 nodes, and one step past the last
     static constexpr int NPOS = (DUP ? 2 * NB : NB) + 8;
+    // Table rows that a batch can read: both sets padded (n0 and n1 nodes, NB in all or,
+    // where a node can be in both, NB each: NB + 4 and 2 NB rows at most) and 4 more.
+    static constexpr int rows_read()
+    {
+        int most = 0;
+        for (int n0 = 0; n0 <= NB; ++n0)
+            for (int n1 = 0; n1 <= (DUP ? NB : NB - n0); ++n1) {
+                const int rows = (n0 + 3) / 4 * 4 + (n1 + 3) / 4 * 4;
+                most = rows > most ? rows : most;
+            }
+        return most + 4;
+    }
     static constexpr int RS = P <= 20 ? 20 : 24;        // row / column weight table stride
     // one table row per batch position: plane weights [0, 16), row weights times the
     // coefficient (re, im) from O_B1, column weights from O_B2; 80 floats, so the
@@ -371,10 +383,8 @@ __global__ __launch_bounds__(kMfmaThreads<R>, (kMfmaPerCu<R, W> * kMfmaThreads<R
                 // (the scheduling barriers keep each step's loads ahead of the
                 // previous step's instructions, which the scheduler would sink
                 // to their uses)
-                // a set's last step reads the operands of one step past it: the two
-                // padded sets fill at most NB + 4 rows (their sizes are multiples of 4
-                // summing to at most NB + 6), so those four rows are inside the table
-                static_assert(S::NB % 4 == 0 && S::NPOS >= S::NB + 8, "one step past the last stays in the table");
+                // a set's last step reads the operands of one step past it
+                static_assert(S::NPOS >= S::rows_read(), "one step past the last stays in the table");
                 Ptrs q = ptrs(k0);
                 Ops o0 = load(q, 0);
                 for (int ks = k0;; ks += 2) {

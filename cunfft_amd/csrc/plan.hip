@@ -1038,7 +1038,8 @@ int api_adjoint_noalloc_dev(typename Traits<T>::plan *p, const void *f, void *fh
             plan_bins(b, im->geom, (int)sizeof(T), im->config[1], im->compensated)) {
             size_t need = b.bytes_for(p->M_total);
             if (need > kNoAllocScratchBytes) {
-                // the fewest slots: the longest chunks
+                // the fewest slots: the longest chunks (the sums then run in another order
+                // than those of the allocating adjoint)
                 b.chunk_base = kChunkShift;
                 need = b.bytes_for(p->M_total);
             }

@@ -398,11 +398,17 @@ __global__ __launch_bounds__(kTileBlock) void k_bin_chunks(const uint32_t *__res
 //   2D    50021 nodes  332 / 218 / 172 / 164       3D   60001 nodes  510 /  423 /  437 /  471
 //   2D   100800 nodes  220 / 220 / 242 / 242       3D  400009 nodes 1090 / 1029 / 1062 / 1169
 //   2D   262144 nodes  182 / 188 / 211 / 222       3D  262145 nodes  646 /  643 /  705 /  797
-// Hence about 1024 chunks at most from splitting in 2D, and 128 nodes or more in 3D,
-// whose slots are larger: there only where no evenly filled tile is split (at 123 nodes
-// per tile, where a third would be, 342 us instead of 293).  A batch has its problems
-// to fill the GPU: the longest chunks.  1D, a node per lane: 64 nodes a chunk while that
-// is at most 512 chunks.
+// Hence about 1024 chunks at most from splitting in 2D (50021 nodes, which that gives 64
+// per chunk, would gain 5% more with 32; a line that lets them have 32 costs 100800
+// radial nodes 10%), and 128 nodes or more in 3D, whose slots are larger: there only
+// where no evenly filled tile is split (at 123 nodes per tile, where a third would be,
+// 342 us instead of 293).  A batch has its problems to fill the GPU: the longest chunks.
+// 1D, a node per lane; the line is flat (m = 4, FP64):
+//   2^16 cells, 32768 nodes   40 /  40 /  41 /  46   clustered     40 /  40 /  41 /  42
+//   2^16 cells, 65536 nodes   42 /  43 /  47 /  53   clustered     41 /  42 /  44 /  49
+//   2^20 cells, 40000 nodes   74 /  74 /  74 /  74   clustered     84 /  81 /  79 /  80
+//   2^20 cells, 90000 nodes   75 /  74 /  75 /  79   clustered     90 /  83 /  82 /  86
+// 64 nodes while that is at most 512 chunks, 128 up to as many, then 256.
 static int plan_chunk_base(int d, int64_t M, int64_t ntiles)
 {
     if (d == 1) return M <= 32768 ? 6 : M <= 65536 ? 7 : kChunkShift;
@@ -426,7 +432,8 @@ static int plan_chunk_base(int d, int64_t M, int64_t ntiles)
 //   FP32 / FP64 128 x 64 x 64 grid, 122881 nodes, m = 4   93 / 117, 100 / 134, 115 / 157
 //   FP64 256 x 64 x 64 grid, 245761 nodes, m = 3         133 /  138 /  153
 // So two from 4096 tiles on (8 chains and more per resident FP64 workgroup), four for
-// FP64 from 16384; below, the chains leave workgroups idle at the end.
+// FP64 from 16384; below, the chains leave workgroups idle at the end in most cases (the
+// FP32 64^3 grid alone would gain: its 700 chunks are fewer than the resident workgroups).
 static int plan_seg_shift(int elem_bytes, int64_t ntiles)
 {
     return ntiles < 4096 ? 0 : elem_bytes == 8 && ntiles >= 16384 ? 2 : 1;

@@ -84,9 +84,7 @@ template <> __device__ __forceinline__ double win_exp<double>(double v) { return
 // z = 1, above it one exponential for both hyperbolic functions, and sin and cos from
 // one reduction by multiples of pi (a node's taps have |s| <= m + 3/2, so z is at most
 // 2 pi sqrt(3m + 9/4) there: 33 for m <= 8, 45 for m = 16).
-// Nodes set, forward and adjoint of 50021 2D nodes, m = 3, FP32: 171 -> 146 us; ten
-// CGNR iterations over 100800 2D nodes, m = 4, FP64: 5.2 -> 3.85 ms (with the
-// chunk rule of binning.hip).
+// Nodes set, forward and adjoint of 50021 2D nodes, m = 3, FP32: 171 -> 146 us.
 // A larger z comes only from a node without a position (window_cell): weight
 // zero, or NaN for a non-finite one.
 constexpr int kKbZMax = 256;

@@ -101,10 +101,9 @@ template <typename T> __device__ __forceinline__ T kb_series(T q)
 
 // sinh(z) / z for 1 < z <= b m (b < 2 pi, m <= 16: below 101).  FP32: the hardware
 // exp2 of the rounded z log2(e), times what the rounding left.
-//  * exp(z) leaves the FP32 range at z = 88.7, where sinh(z) / z does not yet (m = 15
-//    and 16 at an oversampling of 4.5 and more get there), so it is taken at an eighth:
-//    hi - 3 is exact for hi >= 1.44 (and must not be contracted with the product, of
-//    which lo is the rest).
+//  * exp(z) leaves the FP32 range at z = 88.7, sinh(z) at 89.4 (m = 15 and 16 at an
+//    oversampling of 4.5 and more get there), so e is exp(z) / 2: hi - 1 is exact for
+//    hi >= 1.44 (and must not be contracted with the product, of which lo is the rest).
 //  * log2(e) is rounded down for hi, so lo is positive and what is past the range is
 //    infinite, not NaN.
 __device__ __forceinline__ float kb_sinhc(float z)
@@ -112,9 +111,9 @@ __device__ __forceinline__ float kb_sinhc(float z)
 #pragma clang fp contract(off)
     const float hi = z * 1.44269490f;
     const float lo = fmaf(z, 1.92596299e-8f, fmaf(z, 1.44269504f, -hi));   // log2(e) in two parts
-    const float x = __builtin_amdgcn_exp2f(hi - 3.f);
+    const float x = __builtin_amdgcn_exp2f(hi - 1.f);
     const float e = fmaf(x, lo * 0.693147181f, x);
-    return 4.f * (e - 0x1p-6f / e) / z;
+    return (e - 0.25f / e) / z;
 }
 __device__ __forceinline__ double kb_sinhc(double z)
 {

@@ -205,6 +205,10 @@ template <typename T> static void free_device(typename Traits<T>::plan *p)
 }
 
 // src/cunfft.cu:262-280: allocate and zero the device arrays.
+// A memset returns to the host before it has run, and neither the plan's stream
+// nor a caller's waits for the null stream: cleared there, an array could lose
+// the values that the next call copies into it.  So the plan's own stream clears
+// them and is waited for.
 template <typename T> static void init_device_para(typename Traits<T>::plan *p)
 {
     using C2 = typename Traits<T>::hc;
@@ -213,10 +217,12 @@ template <typename T> static void init_device_para(typename Traits<T>::plan *p)
     CUNFFT_HIP(hipMalloc((void **)&p->fhat_gpu, sizeof(C2) * p->N_total));
     CUNFFT_HIP(hipMalloc((void **)&p->x_gpu, sizeof(double) * p->M_total * p->d));
     CUNFFT_HIP(hipMalloc((void **)&p->f_gpu, sizeof(C2) * p->M_total));
-    CUNFFT_HIP(hipMemset(p->g_gpu, 0, sizeof(C2) * p->n_total));
-    CUNFFT_HIP(hipMemset(p->fhat_gpu, 0, sizeof(C2) * p->N_total));
-    CUNFFT_HIP(hipMemset(p->x_gpu, 0, sizeof(double) * p->M_total * p->d));
-    CUNFFT_HIP(hipMemset(p->f_gpu, 0, sizeof(C2) * p->M_total));
+    const hipStream_t s = p->impl ? static_cast<Impl<T> *>(p->impl)->stream : nullptr;
+    CUNFFT_HIP(hipMemsetAsync(p->g_gpu, 0, sizeof(C2) * p->n_total, s));
+    CUNFFT_HIP(hipMemsetAsync(p->fhat_gpu, 0, sizeof(C2) * p->N_total, s));
+    CUNFFT_HIP(hipMemsetAsync(p->x_gpu, 0, sizeof(double) * p->M_total * p->d, s));
+    CUNFFT_HIP(hipMemsetAsync(p->f_gpu, 0, sizeof(C2) * p->M_total, s));
+    CUNFFT_HIP(hipStreamSynchronize(s));
     if (p->impl) {
         Impl<T> *im = static_cast<Impl<T> *>(p->impl);
         im->nodes_changed();

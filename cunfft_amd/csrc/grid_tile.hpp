@@ -4,7 +4,7 @@
 // Forward gridding f_j = sum_l g_l phi(x_j - l/n) (src/cunfft_kernel.cu:514-1093)
 // and adjoint gridding g_l = sum_j f_j phi(x_j - l/n) (src/cunfft_kernel.cu:
 // 608-1197), one workgroup per chunk of the nodes binned to one grid tile
-// (bin.hip).  The window of a node covers W = 2m+2 cells per axis; its cells
+// (binning.hip).  The window of a node covers W = 2m+2 cells per axis; its cells
 // in the padded tile held in LDS are visited one plane (leading-axis index) at
 // a time, with the lanes of a wavefront spread over the W rows x window width
 // of the plane:
